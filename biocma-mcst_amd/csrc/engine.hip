@@ -1175,9 +1175,11 @@ int commit(mcst_engine* e) {
   if ((rc = dev_alloc(e, (void**)&b.sub_divs, T_max * b.nsub * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&e->d_runs, (size_t)RC * sizeof(RunDev)))) return rc;
   if ((rc = dev_alloc(e, (void**)&e->d_rs, (size_t)RC * sizeof(RunState)))) return rc;
+  b.n_shard = run_shards(RC);
+  if ((rc = dev_alloc(e, (void**)&b.shards, (size_t)RC * b.n_shard * sizeof(RunShard)))) return rc;
   if ((rc = dev_alloc(e, (void**)&e->d_comp, (size_t)(RC + 1) * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.rm_tile_off, (RC + 1) * sizeof(uint32_t)))) return rc;
-  if ((rc = dev_alloc(e, (void**)&b.ticket, (1 + RESOLVE_TICKETS) * sizeof(uint32_t)))) return rc;
+  if ((rc = dev_alloc(e, (void**)&b.ticket, (1 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)))) return rc;
   const RequestLevels lv = request_levels(T_max, b.nsub);
   if ((rc = dev_alloc(e, (void**)&b.div_l1, lv.n1 * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.div_l2, lv.n2 * sizeof(uint32_t)))) return rc;
@@ -1185,12 +1187,13 @@ int commit(mcst_engine* e) {
   HIP_TRY(hipMemset(b.div_l1, 0, lv.n1 * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.div_l2, 0, lv.n2 * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.div_l3, 0, lv.n3 * sizeof(uint32_t)));
-  HIP_TRY(hipMemset(b.ticket, 0, (1 + RESOLVE_TICKETS) * sizeof(uint32_t)));
+  HIP_TRY(hipMemset(b.ticket, 0, (1 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.rm_tile_off, 0, (RC + 1) * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.tile_off, 0, (RC + 1) * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.sub_moves, 0, T_max * b.nsub * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.sub_divs, 0, T_max * b.nsub * sizeof(uint32_t)));
   HIP_TRY(hipMemset(e->d_rs, 0, (size_t)RC * sizeof(RunState)));
+  HIP_TRY(hipMemset(b.shards, 0, (size_t)RC * b.n_shard * sizeof(RunShard)));
   b.runs = e->d_runs;
   b.rs = e->d_rs;
   b.comp_off = e->d_comp;

@@ -26,6 +26,7 @@ constexpr uint32_t NSUB_MAX = TILE / 128;  // sub-chunks (the pass's unit of wor
 constexpr uint32_t WAVES = BLOCK / 64;
 constexpr uint32_t RESOLVE_GROUP_MAX = 64;  // sub-chunks per group of the resolve kernel: 32 or 64 (at most 256)
 constexpr uint32_t RESOLVE_TICKETS = 64;    // sub-counters of the resolve kernel's done-count
+constexpr uint32_t TICKET_STRIDE = 32;      // words between two of those counters (a line each)
 constexpr uint32_t DIV_STAGE = 16;          // division requests per sub-chunk divided in the particle pass
 constexpr int MAX_PARAMS = 16;
 constexpr int MAX_VAR = 16;
@@ -180,10 +181,25 @@ struct RunState {
   uint32_t clock_div;
   uint32_t clock_hyd;
   uint32_t pad;
-  unsigned long long step_exits, step_deaths, step_moves, step_requests, step_processed;
   unsigned long long counters[C_COUNT];
   unsigned long long probe_exit_n, probe_div_n;
 };
+
+// One of a run's counter shards: the events of the step under way, added by
+// the blocks whose index falls on the shard and taken (and cleared) by the
+// books.  A line each: atomics on one line are served one after another, about
+// 10 ns each across the XCDs, so 2700 waves adding their moves and particles
+// to two counters of one line took 25 us of a 345 679-particle pass of 41 us.
+// Particles processed need no count: they are the run's Idle slots, n -
+// inactive.
+struct RunShard {
+  unsigned long long moves_requests;  // moves in the low 32 bits, division requests in the high
+  unsigned long long exits_deaths;    // exits low, deaths high
+  unsigned long long pad[14];
+};
+// Shards per run: fewer where many runs spread the atomics anyway (a power of
+// two, at most 16: the books sum a run's shards within 16 lanes).
+constexpr uint32_t run_shards(uint32_t runs) { return runs <= 16 ? 16u : runs <= 256 ? 4u : 1u; }
 
 // Everything a step's kernels receive.
 struct BatchDev {
@@ -209,7 +225,7 @@ struct BatchDev {
   uint32_t* div_l1;
   uint32_t* div_l2;
   uint32_t* div_l3;
-  uint32_t* ticket;         // [1 + RESOLVE_TICKETS] resolve blocks that are done (the last keeps the books)
+  uint32_t* ticket;         // [1 + RESOLVE_TICKETS][TICKET_STRIDE] resolve blocks that are done (the last keeps the books)
   uint32_t* rm_tile_off;    // [R+1] removal layout: first global tile of each run's [0, n_end)
   // per-tile bookkeeping of the removal
   uint32_t* tile_gap;
@@ -232,9 +248,11 @@ struct BatchDev {
   // runs
   const RunDev* runs;
   RunState* rs;
+  RunShard* shards;         // [R][n_shard]
   const MapDev* maps;
   const uint32_t* comp_off; // [R+1]
   uint32_t R;
+  uint32_t n_shard;
   uint32_t n_comp_total;
   uint32_t ns_max;          // largest species count of the batch
   uint32_t T_max;

@@ -317,19 +317,14 @@ __global__ void __launch_bounds__(256) k_transport(BatchDev b) {
 }
 
 // ------------------------------------------------------------------ particles
-// Counters of the tiles a block processed for one run, flushed with one
-// atomic each when the block moves on to another run (or finishes).
-struct TileCounts {
-  uint32_t exits = 0, deaths = 0, moves = 0, requests = 0, processed = 0;
-};
+// This block's counter shard of run r.
+__device__ __forceinline__ RunShard* run_shard(const BatchDev& b, uint32_t r) {
+  return b.shards + (size_t)r * b.n_shard + (blockIdx.x & (b.n_shard - 1u));
+}
 
-__device__ __forceinline__ void flush_counts(RunState* rs, TileCounts& c) {
-  if (c.exits) atomicAdd(&rs->step_exits, (unsigned long long)c.exits);
-  if (c.deaths) atomicAdd(&rs->step_deaths, (unsigned long long)c.deaths);
-  if (c.moves) atomicAdd(&rs->step_moves, (unsigned long long)c.moves);
-  if (c.requests) atomicAdd(&rs->step_requests, (unsigned long long)c.requests);
-  if (c.processed) atomicAdd(&rs->step_processed, (unsigned long long)c.processed);
-  c = TileCounts{};
+// Two counts of a run in one word of its shard (no atomic for none).
+__device__ __forceinline__ void add_pair(unsigned long long* w, uint32_t lo, uint32_t hi) {
+  if (lo | hi) atomicAdd(w, (unsigned long long)lo | ((unsigned long long)hi << 32));
 }
 
 // Adds a block's LDS contribution accumulator, [n_s][win] for compartments
@@ -577,9 +572,15 @@ __global__ void __launch_bounds__(BLK)
     }
   };
 
-  // per-wave counters of the run cnt_run, flushed when the wave changes runs
-  TileCounts cnt_acc;
+  // the wave's exits and deaths of the run cnt_run, added to its shard when
+  // the wave changes runs (its movers and requests are counted from their
+  // lists by k_resolve, a wave's count there being a block's of 8 to 16 waves)
+  uint32_t cnt_exits = 0, cnt_deaths = 0;
   uint32_t cnt_run = 0xFFFFFFFFu;
+  auto flush_counts = [&]() {
+    if (cnt_run != 0xFFFFFFFFu && lane == 0) add_pair(&run_shard(b, cnt_run)->exits_deaths, cnt_exits, cnt_deaths);
+    cnt_exits = cnt_deaths = 0;
+  };
   // the wave's division requests summed per block of each level of the
   // request counts (div_l1/2/3: blocks of 2^6, 2^12, 2^18 sub-chunks),
   // added with one atomic when the wave leaves the block: its sub-chunks
@@ -680,8 +681,7 @@ __global__ void __launch_bounds__(BLK)
     const uint32_t r = cur.r;
     const RunDev& rd = runs[r];
     if (cur.cnt && r != cnt_run) {  // wave moves to another run
-      if (cnt_run != 0xFFFFFFFFu && lane == 0) flush_counts(b.rs + cnt_run, cnt_acc);
-      cnt_acc = TileCounts{};
+      flush_counts();
       cnt_run = r;
     }
     const uint32_t step = rsr[r].step;
@@ -921,12 +921,9 @@ __global__ void __launch_bounds__(BLK)
     // ---- counters of the sub-chunk (wave-uniform)
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
-      cnt_acc.processed += (uint32_t)__popcll(__ballot(idle[j]));
-      cnt_acc.exits += (uint32_t)__popcll(__ballot(exited[j]));
-      cnt_acc.deaths += (uint32_t)__popcll(__ballot(dead[j]));
+      if constexpr (LV) cnt_exits += (uint32_t)__popcll(__ballot(exited[j]));
+      if constexpr (M::CAN_DIE) cnt_deaths += (uint32_t)__popcll(__ballot(dead[j]));
     }
-    cnt_acc.moves += n_mov;
-    cnt_acc.requests += n_div;
 
     __builtin_amdgcn_sched_barrier(0);
     cur = nxt;
@@ -946,7 +943,7 @@ __global__ void __launch_bounds__(BLK)
       flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
     }
   }
-  if (cnt_run != 0xFFFFFFFFu && lane == 0) flush_counts(b.rs + cnt_run, cnt_acc);
+  flush_counts();
 #pragma unroll
   for (int lvl = 0; lvl < 3; ++lvl) flush_requests(lvl);
 }
@@ -963,39 +960,77 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
   constexpr uint32_t NT = 256, NWV = NT / 64;
   __shared__ uint32_t s_w[NWV], s_wl[NWV];
   __shared__ uint32_t s_carry, s_carry_l;
+  __shared__ unsigned long long s_mr[NT], s_ed[NT];  // the counts of 256 runs, summed over their shards
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   if (tid == 0) s_carry = s_carry_l = 0;
-  __syncthreads();
+  const uint32_t nsh = b.n_shard;
   for (uint32_t r0 = 0; r0 < b.R; r0 += NT) {
     const uint32_t r = r0 + tid;
+    // what the books read of the run's state, requested before the shards so
+    // that both round trips to memory overlap
+    RunState* const rs = b.rs + r;
+    uint32_t n = 0, inactive0 = 0, step0 = 0, active = 0;
+    uint32_t cap = 0, div_cap = 0, leave = 0, target = 0;
+    uint64_t min_removal = 0;
+    double ratio = 0.0;
+    unsigned long long cnt[C_COUNT] = {};
+    if (r < b.R) {
+      const RunDev& rd = runs[r];
+      n = rs->n;
+      inactive0 = rs->inactive;
+      step0 = rs->step;
+      active = rs->active;
+#pragma unroll
+      for (int k = 0; k < C_COUNT; ++k) cnt[k] = rs->counters[k];
+      cap = rd.cap;
+      div_cap = rd.div_cap;
+      leave = rd.enable_leave;
+      target = rd.step_target;
+      min_removal = rd.min_removal;
+      ratio = rd.ratio;
+    }
+    // read and reset with atomics: other blocks added to the shards with
+    // atomics up to a moment ago.  One lane per shard, all in flight at once
+    const uint32_t n_run = b.R - r0 < NT ? b.R - r0 : NT;
+    for (uint32_t i0 = 0; i0 < n_run * nsh; i0 += NT) {
+      const uint32_t i = i0 + tid;
+      unsigned long long mr = 0, ed = 0;
+      if (i < n_run * nsh) {
+        RunShard* sh = b.shards + (size_t)r0 * nsh + i;
+        mr = atomicExch(&sh->moves_requests, 0ull);
+        ed = atomicExch(&sh->exits_deaths, 0ull);
+      }
+      // both halves stay below 2^32 (a run has fewer slots): no carry between them
+      for (uint32_t d = nsh >> 1; d; d >>= 1) {
+        mr += __shfl_xor(mr, (int)d, 64);
+        ed += __shfl_xor(ed, (int)d, 64);
+      }
+      if (i < n_run * nsh && i % nsh == 0) {
+        s_mr[i / nsh] = mr;
+        s_ed[i / nsh] = ed;
+      }
+    }
+    __syncthreads();
     uint32_t tiles = 0;   // tiles of [0, n_end) when the run compacts
     uint32_t tiles_l = 0; // tiles of the next step's layout
     if (r < b.R) {
-      RunState* rs = b.rs + r;
-      const RunDev& rd = runs[r];
-      uint32_t step_now, n_now;  // after this step's books
-      if (rs->active) {
-        const uint32_t n = rs->n;
-        // read and reset with atomics: the resolve kernel's blocks added to
-        // the exit counter with atomics up to a moment ago
-        const unsigned long long req = atomicExch(&rs->step_requests, 0ull);
-        const unsigned long long exits = atomicExch(&rs->step_exits, 0ull);
-        const unsigned long long deaths = atomicExch(&rs->step_deaths, 0ull);
-        const unsigned long long moves = atomicExch(&rs->step_moves, 0ull);
-        const unsigned long long processed = atomicExch(&rs->step_processed, 0ull);
-        const uint32_t room = rd.cap - n;
-        const uint32_t budget = room < rd.div_cap ? room : rd.div_cap;
+      uint32_t step_now = step0, n_now = n;  // after this step's books
+      if (active) {
+        const unsigned long long moves = (uint32_t)s_mr[tid], req = s_mr[tid] >> 32;
+        const unsigned long long exits = (uint32_t)s_ed[tid], deaths = s_ed[tid] >> 32;
+        const unsigned long long processed = n - inactive0;  // every Idle slot
+        const uint32_t room = cap - n;
+        const uint32_t budget = room < div_cap ? room : div_cap;
         const uint32_t births = req < budget ? (uint32_t)req : budget;
-        unsigned long long* cnt = rs->counters;
         cnt[C_BIRTHS] += births;
         cnt[C_EXITS] += exits;
         cnt[C_DEATHS] += deaths;
         cnt[C_MOVES] += moves;
         cnt[C_OVERFLOW] += req - births;
         cnt[C_PROCESSED] += processed;
-        uint64_t inactive = (uint64_t)rs->inactive + exits + deaths;
-        const uint64_t thr_ratio = (uint64_t)((double)n * rd.ratio);
-        const uint64_t thr = rd.min_removal > thr_ratio ? rd.min_removal : thr_ratio;
+        uint64_t inactive = (uint64_t)inactive0 + exits + deaths;
+        const uint64_t thr_ratio = (uint64_t)((double)n * ratio);
+        const uint64_t thr = min_removal > thr_ratio ? min_removal : thr_ratio;
         const uint32_t n_end = n + births;
         uint32_t n_keep = n_end, compact = 0;
         if ((b.stages & STAGE_REMOVE) && inactive > thr) {
@@ -1010,29 +1045,28 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
           }
           inactive = 0;
         }
-        const uint32_t step = rs->step + 1u;
         // the age clocks tick with the stages the step ran
         if (b.stages & STAGE_MODEL) rs->clock_div += 1u;
-        if (rd.enable_leave && (b.stages & STAGE_LEAVE)) rs->clock_hyd += 1u;
+        if (leave && (b.stages & STAGE_LEAVE)) rs->clock_hyd += 1u;
+        step_now = step0 + 1u;
+        n_now = n_keep;
         rs->n_end = n_end;
         rs->n_keep = n_keep;
         rs->compact = compact;
         rs->births = births;
         rs->inactive = (uint32_t)inactive;
         rs->n = n_keep;
-        rs->step = step;
-        cnt[C_STEPS] = step;
+        rs->step = step_now;
+        cnt[C_STEPS] = step_now;
         cnt[C_N] = n_keep;
         cnt[C_INACTIVE] = (uint32_t)inactive;
-        step_now = step;
-        n_now = n_keep;
+#pragma unroll
+        for (int k = 0; k < C_COUNT; ++k) rs->counters[k] = cnt[k];
       } else {
         rs->compact = 0;
-        step_now = rs->step;
-        n_now = rs->n;
       }
       if (layout) {  // layout_pass's table, from the values at hand
-        const uint32_t act = step_now < rd.step_target ? 1u : 0u;
+        const uint32_t act = step_now < target ? 1u : 0u;
         tiles_l = act ? (n_now + TILE - 1u) / TILE : 0u;
         rs->active = act;
         rs->n_tiles = tiles_l;
@@ -1076,7 +1110,7 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
   for (uint32_t i = tid; i < (n_sc + 63u) >> 6; i += NT) b.div_l1[i] = 0u;
   for (uint32_t i = tid; i < (n_sc + 4095u) >> 12; i += NT) b.div_l2[i] = 0u;
   for (uint32_t i = tid; i <= (n_sc >> 18); i += NT) b.div_l3[i] = 0u;
-  for (uint32_t i = tid; i <= RESOLVE_TICKETS; i += NT) b.ticket[i] = 0u;
+  for (uint32_t i = tid; i <= RESOLVE_TICKETS; i += NT) b.ticket[i * TICKET_STRIDE] = 0u;
 }
 
 // After the particle pass, per group of 32 or 64 sub-chunks (one per thread
@@ -1158,6 +1192,7 @@ __global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __res
   uint32_t GS = 32;
   while (GS < RES_SC && (n_sc + 2 * GS - 1) / (2 * GS) >= n_res) GS *= 2;
   const uint32_t n_groups = (n_sc + GS - 1) / GS;
+  uint32_t ev_run = 0, ev_moves = 0, ev_req = 0;  // movers and requests of the block's groups (thread 0)
   const bool leave_stage = (b.stages & STAGE_LEAVE) != 0;
   if (tr_block) {
     if constexpr (ROWS)
@@ -1200,6 +1235,22 @@ __global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __res
     __syncthreads();
     // ---- movers
     const uint32_t total = s_pre[GS];
+    // the step's moves and requests, from the lists: one atomic per block and
+    // run, or per sub-chunk where the group holds several runs
+    const uint32_t g_last = n_sc - sc0 < GS ? n_sc - sc0 - 1u : GS - 1u;
+    if (s_run[0] == s_run[g_last]) {
+      if (tid == 0) {
+        if (s_run[0] != ev_run) {
+          add_pair(&run_shard(b, ev_run)->moves_requests, ev_moves, ev_req);
+          ev_run = s_run[0];
+          ev_moves = ev_req = 0;
+        }
+        ev_moves += total;
+        ev_req += s_dpre[GS];
+      }
+    } else if (tid <= g_last) {
+      add_pair(&run_shard(b, s_run[tid])->moves_requests, s_pre[tid + 1] - s_pre[tid], s_dpre[tid + 1] - s_dpre[tid]);
+    }
     for (uint32_t e = tid; e < total; e += blockDim.x) {
       uint32_t lo = 0, hi = GS;  // the sub-chunk j with s_pre[j] <= e < s_pre[j+1]
       while (hi - lo > 1) {
@@ -1259,9 +1310,9 @@ __global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __res
       // queued tens of thousands of them on one address per step
       const uint32_t r_lead = __builtin_amdgcn_readfirstlane(r);
       const uint64_t ex_lead = __ballot(exits && r == r_lead);
-      if (exits && r != r_lead) atomicAdd(&rs->step_exits, 1ull);
+      if (exits && r != r_lead) add_pair(&run_shard(b, r)->exits_deaths, 1u, 0u);
       if (ex_lead && lane == (uint32_t)__ffsll((long long)ex_lead) - 1u)
-        atomicAdd(&b.rs[r_lead].step_exits, (unsigned long long)__popcll(ex_lead));
+        add_pair(&run_shard(b, r_lead)->exits_deaths, (uint32_t)__popcll(ex_lead), 0u);
     }
     // ---- divisions: every request of the group at once, one thread each
     const uint32_t n_req = s_dpre[GS];
@@ -1349,15 +1400,18 @@ __global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __res
     }
     __syncthreads();
   }
+  if (tid == 0) add_pair(&run_shard(b, ev_run)->moves_requests, ev_moves, ev_req);
   // ---- the last block to finish keeps the books.  The books read, of this
-  // kernel's work, only the exit counters, which are updated by atomics:
+  // kernel's work, only the counter shards, which are updated by atomics:
   // every thread waits for its memory operations to complete before its
   // block counts itself done, and the last block reads the counters with
   // atomics.  No cache writeback is needed (an agent-scope fence per block
   // writes back this XCD's L2 each time: 60 us over a 2048-block grid).
-  // Blocks count themselves done on RESOLVE_TICKETS sub-counters (block b on
-  // b % RESOLVE_TICKETS), and the last of each on the main counter, so no counter
-  // takes more than a few dozen atomics; resolve blocks without a group take no
+  // Up to RESOLVE_TICKETS blocks count themselves done on one counter (under
+  // 1 us of atomics one after another, about what a second level costs); more
+  // on RESOLVE_TICKETS sub-counters (block b on b % RESOLVE_TICKETS), a line
+  // each, and the last of each on the main counter, so no line takes more than
+  // a few dozen atomics; resolve blocks without a group take no
   // part, transport blocks do (the books advance the step count they read).
   const uint32_t nb = n_groups < n_res ? n_groups : n_res;  // resolve blocks with work
   const uint32_t np = nb + tr_blocks;                       // blocks that count themselves done
@@ -1370,11 +1424,15 @@ __global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __res
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (tid == 0) {
-    const uint32_t j = id % RESOLVE_TICKETS;
-    const uint32_t in_j = (np - j + RESOLVE_TICKETS - 1u) / RESOLVE_TICKETS;  // blocks counting on sub-counter j
-    const uint32_t n_sub = np < RESOLVE_TICKETS ? np : RESOLVE_TICKETS;        // sub-counters in use
     uint32_t last = 0;
-    if (atomicAdd(b.ticket + 1u + j, 1u) == in_j - 1u) last = atomicAdd(b.ticket, 1u) == n_sub - 1u ? 1u : 0u;
+    if (np <= RESOLVE_TICKETS) {
+      last = atomicAdd(b.ticket, 1u) == np - 1u ? 1u : 0u;
+    } else {
+      const uint32_t j = id % RESOLVE_TICKETS;
+      const uint32_t in_j = (np - j + RESOLVE_TICKETS - 1u) / RESOLVE_TICKETS;  // blocks counting on sub-counter j
+      if (atomicAdd(b.ticket + (1u + j) * TICKET_STRIDE, 1u) == in_j - 1u)
+        last = atomicAdd(b.ticket, 1u) == RESOLVE_TICKETS - 1u ? 1u : 0u;
+    }
     s_last = last;
   }
   __syncthreads();
