@@ -461,6 +461,8 @@ struct mcst_engine {
   int grid_particle = 1, grid_transport = 1;
   mcst::ParticleLaunch plaunch;
   int tuned_block = 0;              // particle-pass shape chosen by mcst_engine_autotune (0: none)
+  void* export_mem = nullptr;       // device side of the export reads (EXPORT_KEEP bytes at most), kept between them
+  size_t export_bytes = 0;
   void* sort_mem = nullptr;         // scratch of the particle reorder, sized for sort_n slots
   uint64_t sort_n = 0;
   size_t sort_temp = 0;
@@ -547,6 +549,9 @@ void release(mcst_engine* e) {
   e->alt_state = e->alt_age_hyd = e->alt_age_div = nullptr;
   e->alt_clk_hyd = e->alt_clk_div = nullptr;
   e->alt_P = 0;
+  if (e->export_mem) (void)hipFree(e->export_mem);
+  e->export_mem = nullptr;
+  e->export_bytes = 0;
   if (e->sort_mem) (void)hipFree(e->sort_mem);
   e->sort_mem = nullptr;
   e->sort_n = 0;
@@ -2397,20 +2402,51 @@ int mcst_run_get_contributions(mcst_engine* e, int32_t run, double* S) { return 
 int mcst_run_get_gas_concentrations(mcst_engine* e, int32_t run, double* C) { return get_liquid(e, run, C, 3); }
 int mcst_run_get_gas_mass(mcst_engine* e, int32_t run, double* m) { return get_liquid(e, run, m, 4); }
 
+// Device memory of an export read: the engine's kept buffer, or for more than
+// EXPORT_KEEP bytes an allocation of the call's own.  (An allocation and its
+// free took about 0.1 ms of each read.)  The engine's reads run one at a time
+// and end with the stream idle, so they can share the buffer.
+namespace {
+constexpr size_t EXPORT_KEEP = 64ull << 20;
+struct ExportBuffer {
+  void* p = nullptr;
+  bool own = false;
+  ~ExportBuffer() {
+    if (own && p) (void)hipFree(p);
+  }
+  hipError_t get(mcst_engine* e, size_t bytes) {
+    if (bytes > EXPORT_KEEP) {
+      own = true;
+      return hipMalloc(&p, bytes);
+    }
+    if (bytes > e->export_bytes) {
+      if (e->export_mem) (void)hipFree(e->export_mem);
+      e->export_mem = nullptr;
+      e->export_bytes = 0;
+      const hipError_t err = hipMalloc(&e->export_mem, bytes);
+      if (err != hipSuccess) return err;
+      e->export_bytes = bytes;
+    }
+    p = e->export_mem;
+    return hipSuccess;
+  }
+};
+}  // namespace
+
 int mcst_run_get_repartition(mcst_engine* e, int32_t run, uint64_t* hist) {
   CHECK_READY(e, run);
   if (!hist) return fail(MCST_ERR_ARG, "null output");
   const uint32_t n_c = e->h_runs[run].n_c;
-  unsigned long long* d = nullptr;
-  HIP_TRY(hipMalloc(&d, n_c * sizeof(unsigned long long)));
+  ExportBuffer buf;
+  HIP_TRY(buf.get(e, n_c * sizeof(unsigned long long)));
+  unsigned long long* d = (unsigned long long*)buf.p;
   hipError_t err = hipMemsetAsync(d, 0, n_c * sizeof(unsigned long long), e->stream);
   if (err == hipSuccess) {
-    launch_repartition(e->bd, (uint32_t)run, d, e->stream);
+    launch_repartition(e->bd, (uint32_t)run, n_c, d, e->stream);
     err = hipGetLastError();
   }
   if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
   if (err == hipSuccess) err = hipMemcpy(hist, d, n_c * sizeof(uint64_t), hipMemcpyDeviceToHost);
-  (void)hipFree(d);
   if (err != hipSuccess) return fail(MCST_ERR_DEVICE, std::string("repartition: ") + hipGetErrorString(err));
   return MCST_OK;
 }
@@ -2464,7 +2500,7 @@ int mcst_run_get_repartition_noalloc(mcst_engine* e, int32_t run, uint64_t* hist
   if (rc) return rc;
   // the array keeps the last call's counts: clear the run's n_c counters
   launch_clear_u64(d, n_c, e->stream);
-  launch_repartition(e->bd, (uint32_t)run, d, e->stream);
+  launch_repartition(e->bd, (uint32_t)run, n_c, d, e->stream);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(hist, d, n_c * sizeof(uint64_t), hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(hipStreamSynchronize(e->stream));
@@ -2481,19 +2517,18 @@ int mcst_run_get_properties(mcst_engine* e, int32_t run, double* values, double*
   const uint64_t rows = (uint64_t)e->model->nv + 1, n = s.n;
   // the per-particle values take device memory only when they are asked for
   const size_t vb = values ? rows * n * sizeof(double) : 0, sb = rows * d.n_c * sizeof(double);
-  char* buf = nullptr;
-  HIP_TRY(hipMalloc((void**)&buf, vb + sb + 8));
-  double* dv = values ? (double*)buf : nullptr;
-  double* ds = (double*)(buf + vb);
+  ExportBuffer buf;
+  HIP_TRY(buf.get(e, vb + sb + 8));
+  double* dv = values ? (double*)buf.p : nullptr;
+  double* ds = (double*)((char*)buf.p + vb);
   hipError_t err = hipMemsetAsync(ds, 0, sb, e->stream);
   if (err == hipSuccess && n) {
-    e->model->ops->properties(e->bd, (uint32_t)run, n, dv, ds, e->stream);
+    e->model->ops->properties(e->bd, (uint32_t)run, n, d.n_c, dv, ds, e->stream);
     err = hipGetLastError();
   }
   if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
   if (err == hipSuccess && values && vb) err = hipMemcpy(values, dv, vb, hipMemcpyDeviceToHost);
   if (err == hipSuccess && spatial) err = hipMemcpy(spatial, ds, sb, hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
   if (err != hipSuccess) return fail(MCST_ERR_DEVICE, std::string("properties: ") + hipGetErrorString(err));
   return MCST_OK;
 }

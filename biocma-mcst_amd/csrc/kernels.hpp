@@ -39,13 +39,14 @@ struct ModelOps {
   // (for the next step's transport, or into S)
   void (*resolve)(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s);
   const void* (*resolve_kernel)();  // for occupancy queries
-  void (*properties)(const BatchDev& b, uint32_t run, uint64_t n, double* values, double* spatial, hipStream_t s);
+  void (*properties)(const BatchDev& b, uint32_t run, uint64_t n, uint32_t n_c, double* values, double* spatial,
+                     hipStream_t s);
 };
 const ModelOps* builtin_model_ops(int model_id);
 
 void launch_removal(const BatchDev& b, uint32_t n_var, int grid, hipStream_t s);
 void launch_layout(const BatchDev& b, hipStream_t s);
-void launch_repartition(const BatchDev& b, uint32_t run, unsigned long long* hist, hipStream_t s);
+void launch_repartition(const BatchDev& b, uint32_t run, uint32_t n_c, unsigned long long* hist, hipStream_t s);
 void launch_clear_u64(unsigned long long* p, uint64_t n, hipStream_t s);
 
 // Stable sort of one run's particles by position (sort.hip).  pos, status

@@ -7,6 +7,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "models.hpp"
 
@@ -1483,34 +1485,93 @@ __device__ void layout_pass(const BatchDev& b) {
 
 
 // ------------------------------------------------------------------ properties
+// One wave's values of one variable added to an LDS accumulator: lanes `in`
+// add x to acc[k].  A wave whose lanes all hold one compartment (particles in
+// compartment order) sums first and adds once.
+__device__ __forceinline__ void add_by_compartment(double* acc, bool in, uint32_t k, bool one, uint32_t k0,
+                                                   uint32_t lane, double x) {
+  if (one) {
+    double t = in ? x : 0.0;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) t += __shfl_xor(t, d, 64);
+    if (lane == 0) atomicAdd(acc + k0, t);
+  } else if (in) {
+    atomicAdd(acc + k, x);
+  }
+}
+
 // Per-particle export values of run r (get_properties, post_process.hpp:54-98):
 // for every Idle slot the model state and M::mass, row-major [n_var+1][n]
 // (zero for inactive slots), and their sums per compartment [n_var+1][n_c].
 // values may be null: the sums only.
+//
+// A block takes a contiguous range of slots and sums them in LDS, then adds
+// its nonzero sums to the device's: with one global atomic per particle and
+// variable instead, the particles of a compartment, which sit together, queued
+// on one address (1e6 particles of 10 values in 500 compartments 1187 us, now
+// 58 us; 1e5 of 3 in 64 compartments 234 us, now 17 us).  LDS holds `vg` variables of `win`
+// compartments; block row y takes one such share (variables y % n_vg, window
+// y / n_vg), reading the positions again for each.
+constexpr uint32_t EXPORT_THREADS = 512;
+constexpr uint32_t EXPORT_LDS = 64 * 1024;      // two blocks per CU
+constexpr uint32_t EXPORT_MIN_SLOTS = 4096;     // per block: 8 rounds of its threads
+constexpr uint32_t EXPORT_MAX_BLOCKS = 512;
+constexpr uint32_t EXPORT_MAX_ROWS = 32768;     // block rows of one launch
 template <class M>
-__global__ void __launch_bounds__(256) k_properties(BatchDev b, uint32_t r, uint64_t n, double* values,
-                                                    double* spatial) {
-  constexpr int NV = M::NV;
+__global__ void __launch_bounds__(EXPORT_THREADS) k_properties(BatchDev b, uint32_t r, uint64_t n, double* values,
+                                                               double* spatial, uint32_t vg, uint32_t n_vg,
+                                                               uint32_t win, uint32_t y0) {
+  constexpr uint32_t NV = M::NV, NT = EXPORT_THREADS;
+  extern __shared__ double s_acc[];  // [vg][w]
   const RunDev& rd = b.runs[r];
   const uint32_t n_c = rd.n_c;
-  for (uint64_t s = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; s < n; s += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t g = rd.p_off + s;
-    if (b.status[g] != IDLE) {
-      if (values)
-        for (int v = 0; v <= NV; ++v) values[(uint64_t)v * n + s] = 0.0;
-      continue;
-    }
-    const uint32_t c = b.pos[g];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t y = y0 + blockIdx.y;
+  const uint32_t v0 = (y % n_vg) * vg, v1 = v0 + vg < NV + 1u ? v0 + vg : NV + 1u;
+  const uint32_t c0 = (y / n_vg) * win, w = n_c - c0 < win ? n_c - c0 : win;
+  const bool store = values && y < n_vg;  // the first window's blocks write the values
+  const bool has_mass = v1 == NV + 1u;
+  const uint64_t per = (n + gridDim.x - 1) / gridDim.x;
+  const uint64_t i0 = blockIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
+  for (uint32_t i = tid; i < (v1 - v0) * w; i += NT) s_acc[i] = 0.0;
+  __syncthreads();
+  double p[M::NP > 0 ? M::NP : 1];
+#pragma unroll
+  for (int q = 0; q < M::NP; ++q) p[q] = rd.params[q];
+  for (uint64_t base = i0; base < i1; base += NT) {
+    const uint64_t s = base + tid;
+    const bool valid = s < i1;
+    const uint64_t g = rd.p_off + (valid ? s : i0);
+    const bool live = valid && b.status[g] == IDLE;
+    const uint32_t k = b.pos[g] - c0;  // wraps above the window when below it
+    const bool in = live && k < w;
+    const uint64_t mask = __ballot(in);
+    const uint32_t lead = mask ? (uint32_t)__ffsll((long long)mask) - 1u : 0u;
+    const uint32_t k0 = (uint32_t)__shfl((int)k, (int)lead, 64);
+    const bool one = mask && __ballot(in && k == k0) == mask;
     double x[NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      x[v] = b.state[(uint64_t)v * b.P + g];
-      if (values) values[(uint64_t)v * n + s] = x[v];
-      unsafeAtomicAdd(spatial + (uint64_t)v * n_c + c, x[v]);
+    for (uint32_t v = 0; v < NV; ++v)
+      x[v] = (has_mass || (v >= v0 && v < v1)) && live ? b.state[(uint64_t)v * b.P + g] : 0.0;
+#pragma unroll
+    for (uint32_t v = 0; v < NV; ++v) {
+      if (v < v0 || v >= v1) continue;
+      if (store && valid) values[(uint64_t)v * n + s] = x[v];
+      add_by_compartment(s_acc + (v - v0) * w, in, k, one, k0, lane, x[v]);
     }
-    const double m = M::mass(rd.params, x);
-    if (values) values[(uint64_t)NV * n + s] = m;
-    unsafeAtomicAdd(spatial + (uint64_t)NV * n_c + c, m);
+    if (has_mass) {
+      const double m = live ? M::mass(p, x) : 0.0;
+      if (store && valid) values[(uint64_t)NV * n + s] = m;
+      add_by_compartment(s_acc + (NV - v0) * w, in, k, one, k0, lane, m);
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < (v1 - v0) * w; i += NT) {
+    const double t = s_acc[i];
+    if (t != 0.0) {
+      const uint32_t q = i / w;
+      unsafeAtomicAdd(spatial + (size_t)(v0 + q) * n_c + c0 + (i - q * w), t);
+    }
   }
 }
 
@@ -1603,8 +1664,18 @@ const void* resolve_kernel_t() {
   return (const void*)&k_resolve<M, false>;
 }
 template <class M>
-void properties_t(const BatchDev& b, uint32_t run, uint64_t n, double* values, double* spatial, hipStream_t s) {
-  hipLaunchKernelGGL(k_properties<M>, dim3(1024), dim3(256), 0, s, b, run, n, values, spatial);
+void properties_t(const BatchDev& b, uint32_t run, uint64_t n, uint32_t n_c, double* values, double* spatial,
+                  hipStream_t s) {
+  constexpr uint32_t NV1 = M::NV + 1;
+  const uint32_t cells = EXPORT_LDS / sizeof(double);
+  const uint32_t win = n_c < cells ? n_c : cells;                      // compartments in LDS
+  const uint32_t vg = cells / win < NV1 ? cells / win : NV1;           // variables in LDS
+  const uint32_t n_vg = (NV1 + vg - 1) / vg, n_win = (uint32_t)(((uint64_t)n_c + win - 1) / win);
+  const uint64_t want = (n + EXPORT_MIN_SLOTS - 1) / EXPORT_MIN_SLOTS;
+  const uint32_t grid = (uint32_t)(want < EXPORT_MAX_BLOCKS ? (want ? want : 1) : EXPORT_MAX_BLOCKS);
+  for (uint32_t y = 0; y < n_vg * n_win; y += EXPORT_MAX_ROWS)
+    hipLaunchKernelGGL(k_properties<M>, dim3(grid, std::min(n_vg * n_win - y, EXPORT_MAX_ROWS)), dim3(EXPORT_THREADS),
+                       (size_t)vg * win * sizeof(double), s, b, run, n, values, spatial, vg, n_vg, win, y);
 }
 
 // The launchers of model M's kernels.
