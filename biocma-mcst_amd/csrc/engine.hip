@@ -484,6 +484,7 @@ struct mcst_engine {
   int tuned_group = -1;
   int grid_move = 1;
   bool removal_possible = true;
+  uint32_t max_tiles = 0;           // largest slot capacity of a run on the device, in tiles
   bool any_leave = true;            // some run on the device has a leaving flow (the pass's leave variant)
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
@@ -867,8 +868,12 @@ int refresh_tables(mcst_engine* e) {
   b.n_comp_total = n_comp;
   b.maps = e->d_maps;
   e->any_leave = false;
-  for (uint32_t r = 0; r < R; ++r)
-    if (e->runs[r].phase == 1 && e->h_runs[r].enable_leave) e->any_leave = true;
+  e->max_tiles = 0;
+  for (uint32_t r = 0; r < R; ++r) {
+    if (e->runs[r].phase != 1) continue;
+    if (e->h_runs[r].enable_leave) e->any_leave = true;
+    e->max_tiles = std::max(e->max_tiles, e->runs[r].tiles);
+  }
   e->removal_possible = e->model->can_die || e->any_leave;
   return choose_launch(e);
 }
@@ -1167,10 +1172,8 @@ int commit(mcst_engine* e) {
   if ((rc = dev_alloc(e, (void**)&b.age_div, P * sizeof(double)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.clk_hyd, P * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.clk_div, P * sizeof(uint32_t)))) return rc;
-  uint32_t** tile_arrays[] = {&b.tile_gap, &b.tile_fill, &b.tile_gap_off, &b.tile_fill_off};
-  for (uint32_t** a : tile_arrays)
-    if ((rc = dev_alloc(e, (void**)a, T_max * sizeof(uint32_t)))) return rc;
-  if ((rc = dev_alloc(e, (void**)&b.fill_src, P * sizeof(uint32_t)))) return rc;
+  if ((rc = dev_alloc(e, (void**)&b.tile_cnt, T_max * sizeof(unsigned long long)))) return rc;
+  if ((rc = dev_alloc(e, (void**)&b.tile_pre, (T_max + 1) * sizeof(unsigned long long)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.tile_off, (RC + 1) * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.move_rec, T_max * TILE * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.div_rec, T_max * TILE * sizeof(uint32_t)))) return rc;
@@ -1184,7 +1187,7 @@ int commit(mcst_engine* e) {
   if ((rc = dev_alloc(e, (void**)&b.shards, (size_t)RC * b.n_shard * sizeof(RunShard)))) return rc;
   if ((rc = dev_alloc(e, (void**)&e->d_comp, (size_t)(RC + 1) * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.rm_tile_off, (RC + 1) * sizeof(uint32_t)))) return rc;
-  if ((rc = dev_alloc(e, (void**)&b.ticket, (1 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)))) return rc;
+  if ((rc = dev_alloc(e, (void**)&b.ticket, (2 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)))) return rc;
   const RequestLevels lv = request_levels(T_max, b.nsub);
   if ((rc = dev_alloc(e, (void**)&b.div_l1, lv.n1 * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.div_l2, lv.n2 * sizeof(uint32_t)))) return rc;
@@ -1192,7 +1195,7 @@ int commit(mcst_engine* e) {
   HIP_TRY(hipMemset(b.div_l1, 0, lv.n1 * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.div_l2, 0, lv.n2 * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.div_l3, 0, lv.n3 * sizeof(uint32_t)));
-  HIP_TRY(hipMemset(b.ticket, 0, (1 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)));
+  HIP_TRY(hipMemset(b.ticket, 0, (2 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.rm_tile_off, 0, (RC + 1) * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.tile_off, 0, (RC + 1) * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.sub_moves, 0, T_max * b.nsub * sizeof(uint32_t)));
@@ -1266,7 +1269,7 @@ void launch_step(mcst_engine* e, uint32_t stages, const hipEvent_t* ev = nullptr
   const uint32_t aux = b.part ? e->part_aux : ahead ? (uint32_t)(e->grid_transport - 1) : 0u;
   ops.resolve(b, e->grid_move, aux, ahead, e->stream);
   mark(3);
-  if (e->removal_possible) launch_removal(b, nv, e->grid_particle, e->stream);
+  if (e->removal_possible) launch_removal(b, nv, e->grid_particle, e->max_tiles, e->stream);
   mark(4);
 }
 
@@ -1465,11 +1468,8 @@ int grow_pool(mcst_engine* e, uint64_t min_tiles) {
       {(void**)&b.div_l1, lv.n1 * 4, 0, 0, nullptr},
       {(void**)&b.div_l2, lv.n2 * 4, 0, 0, nullptr},
       {(void**)&b.div_l3, lv.n3 * 4, 0, 0, nullptr},
-      {(void**)&b.tile_gap, T1 * 4, 0, 0, nullptr},
-      {(void**)&b.tile_fill, T1 * 4, 0, 0, nullptr},
-      {(void**)&b.tile_gap_off, T1 * 4, 0, 0, nullptr},
-      {(void**)&b.tile_fill_off, T1 * 4, 0, 0, nullptr},
-      {(void**)&b.fill_src, P1 * 4, 0, 0, nullptr},
+      {(void**)&b.tile_cnt, T1 * 8, 0, 0, nullptr},
+      {(void**)&b.tile_pre, (T1 + 1) * 8, 0, 0, nullptr},
       {(void**)&b.move_rec, P1 * 4, 0, 0, nullptr},
       {(void**)&b.div_rec, P1 * 4, 0, 0, nullptr},
       {(void**)&b.div_pos, P1 * 4, 0, 0, nullptr},

@@ -13,7 +13,7 @@
 //                    run, mother halving, daughters written to [n, n + births)
 //                    (particles_container.hpp:559-599); its last block keeps the
 //                    books: counters, removal decision (particles_container.hpp:539-557)
-//   k_gap_count / k_gap_scan / k_gap_list / k_gap_fill
+//   k_remove_runs, or k_gap_count and k_gap_fill for large runs
 //                    removal of Exit/Dead slots by gap filling over [0, n + births)
 //                    (particles_container.hpp:292-385,735-796), when a particle
 //                    can become inactive
@@ -30,145 +30,201 @@
 
 namespace mcst {
 
-namespace {
-
-// Exclusive scan of in[0..n) into out (optional) by one block of SCAN_THREADS
-// threads, in ascending or descending index order; returns the total.
-//  - up to RB items per thread: each thread owns a contiguous run, loaded in
-//    one round; one block-wide scan of the per-thread sums;
-//  - more: the items are read in coalesced chunks of SCAN_THREADS (item
-//    base + j*SCAN_THREADS + tid), RB chunks at a time with all their loads
-//    in flight; the waves scan each chunk, publish their totals for all RB
-//    chunks at once, and every thread adds up the totals before it (two
-//    barriers per RB chunks).  One CU streams the 2e5 tile counts of a
-//    2e8-particle run in about 0.1 ms; contiguous runs of 200 items per
-//    thread took 0.45 ms (each load instruction touched 64 lines).
-__device__ uint32_t block_scan(const uint32_t* in, uint32_t* out, uint32_t n, bool descending) {
-  constexpr uint32_t RB = 16;
-  __shared__ uint32_t s_w[RB][SCAN_WAVES];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  if (n <= RB * SCAN_THREADS) {
-    const uint32_t per = (n + SCAN_THREADS - 1) / SCAN_THREADS;
-    const uint32_t k0 = tid * per;
-    const uint32_t k1 = (k0 + per < n) ? k0 + per : n;
-    uint32_t v[RB], sum = 0;
+// ------------------------------------------------------------------ removal
+// Over the slots [0, n_end) of every compacting run: gaps are the non-Idle
+// slots below n_keep (ascending); fillers the Idle slots in [n_keep, n_end)
+// (descending), the step's newborns among them.  The i-th gap receives the
+// i-th filler (while both last, should the inactive count be wrong).
+//
+// The removal is launched with every step of a batch in which particles can
+// leave, and does nothing in most of them (a run compacts when a hundredth of
+// it is inactive), so what it costs is its launches, about 4.5 us each between
+// two others: it used to be four.  Runs of up to REMOVE_RUN_TILES tiles are
+// compacted by one block each, in one launch; above, the status bytes are
+// counted per tile by the whole grid, whose last block adds up the tiles, and
+// a second launch fills the gaps.  A single block compacts 250 000 slots of 8
+// states (1 % of them gaps) in 90 us, in every 50th step or fewer of the
+// lattice tanks: under 2 us a step against the second launch's 4.5; the time
+// grows with the slots, so the line lies at twice that size.  (Launches of a
+// step: 100 000 particles of a ring 26 -> 21 us a step, 250 000 of a lattice
+// 50 -> 44 us, both with four launches before.)
+__device__ __forceinline__ void move_particle(const BatchDev& b, uint32_t n_var, uint64_t dst, uint64_t src) {
+  // every load of a group before its stores: the arrays may alias as far as
+  // the compiler knows, and a load behind each store is a round trip each
+  const uint32_t pos = b.pos[src], ch = b.clk_hyd[src], cd = b.clk_div[src];
+  const double ah = b.age_hyd[src], ad = b.age_div[src];
+  for (uint32_t v0 = 0; v0 < n_var; v0 += 4) {
+    double x[4];
 #pragma unroll
-    for (uint32_t j = 0; j < RB; ++j) {
-      const uint32_t k = k0 + j;
-      v[j] = k < k1 ? in[descending ? n - 1u - k : k] : 0u;
-      sum += v[j];
-    }
-    const uint32_t inc = wave_incl_scan(sum, lane);
-    __syncthreads();  // earlier readers of s_w are done
-    if (lane == 63) s_w[0][wave] = inc;
-    __syncthreads();
-    uint32_t wpre = 0, tot = 0;
-    for (uint32_t w = 0; w < SCAN_WAVES; ++w) {
-      const uint32_t x = s_w[0][w];
-      if (w < wave) wpre += x;
-      tot += x;
-    }
-    if (out) {
-      uint32_t run = wpre + inc - sum;
+    for (uint32_t j = 0; j < 4; ++j) x[j] = v0 + j < n_var ? b.state[(uint64_t)(v0 + j) * b.P + src] : 0.0;
 #pragma unroll
-      for (uint32_t j = 0; j < RB; ++j) {
-        const uint32_t k = k0 + j;
-        if (k < k1) out[descending ? n - 1u - k : k] = run;
-        run += v[j];
-      }
-    }
-    return tot;
+    for (uint32_t j = 0; j < 4; ++j)
+      if (v0 + j < n_var) b.state[(uint64_t)(v0 + j) * b.P + dst] = x[j];
   }
-  uint32_t carry = 0;  // the items before the current chunks (the same in every thread)
-  for (uint32_t base = 0; base < n; base += RB * SCAN_THREADS) {
-    uint32_t v[RB], inc[RB];
-#pragma unroll
-    for (uint32_t j = 0; j < RB; ++j) {
-      const uint32_t k = base + j * SCAN_THREADS + tid;
-      v[j] = k < n ? in[descending ? n - 1u - k : k] : 0u;
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < RB; ++j) inc[j] = wave_incl_scan(v[j], lane);
-    __syncthreads();  // earlier readers of s_w are done
-    if (lane == 63)
-#pragma unroll
-      for (uint32_t j = 0; j < RB; ++j) s_w[j][wave] = inc[j];
-    __syncthreads();
-#pragma unroll
-    for (uint32_t j = 0; j < RB; ++j) {
-      uint32_t wpre = 0, tot = 0;
-      for (uint32_t w = 0; w < SCAN_WAVES; ++w) {
-        const uint32_t x = s_w[j][w];
-        if (w < wave) wpre += x;
-        tot += x;
-      }
-      const uint32_t k = base + j * SCAN_THREADS + tid;
-      if (out && k < n) out[descending ? n - 1u - k : k] = carry + wpre + inc[j] - v[j];
-      carry += tot;
-    }
-  }
-  return carry;
+  b.pos[dst] = pos;
+  b.status[dst] = IDLE;
+  b.age_hyd[dst] = ah;
+  b.age_div[dst] = ad;
+  b.clk_hyd[dst] = ch;
+  b.clk_div[dst] = cd;
 }
 
-}  // namespace
+// One block per run: the gaps from the front, listed in LDS until the next
+// 8192 slots' may not fit (they are sparse: a hundredth of a run fits whole),
+// and the fillers from the back, 4096 slots at a time (nearly all of them),
+// matched as far as the shorter list goes.  (4096 slots of gaps at a time,
+// moved before the next were read, took 335 us for 250 000 slots of 8 states,
+// a round trip per 41 gaps.)
+constexpr uint32_t REMOVE_THREADS = 1024, GAP_LIST = 8 * REMOVE_THREADS, FILL_LIST = 4 * REMOVE_THREADS;
+__global__ void __launch_bounds__(REMOVE_THREADS) k_remove_runs(BatchDev b, uint32_t n_var) {
+  constexpr uint32_t NWV = REMOVE_THREADS / 64;
+  __shared__ uint32_t s_gap[GAP_LIST], s_fill[FILL_LIST];
+  __shared__ uint32_t s_w[NWV];
+  const uint32_t r = blockIdx.x;
+  const RunState* rs = b.rs + r;
+  if (rs->compact != 1u) return;
+  const uint32_t n_end = rs->n_end, n_keep = rs->n_keep;
+  const uint64_t p0 = b.runs[r].p_off;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  // Idle flags of the thread's 4 slots from s0 on that are in [lo, hi)
+  auto idle4 = [&](uint32_t w, uint32_t s0, uint32_t lo, uint32_t hi, bool idle) -> uint32_t {
+    uint32_t f = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const bool hit = s0 + j >= lo && s0 + j < hi && ((((w >> (8 * j)) & 0xFFu) == IDLE) == idle);
+      f |= (hit ? 1u : 0u) << j;
+    }
+    return f;
+  };
+  // block-wide: flags before this thread's, and their total
+  auto scan = [&](uint32_t c, uint32_t& tot) -> uint32_t {
+    const uint32_t inc = wave_incl_scan(c, lane);
+    __syncthreads();  // earlier readers of s_w and of the lists are done
+    if (lane == 63) s_w[wave] = inc;
+    __syncthreads();
+    uint32_t at = inc - c;
+    tot = 0;
+    for (uint32_t k = 0; k < NWV; ++k) {
+      if (k < wave) at += s_w[k];
+      tot += s_w[k];
+    }
+    return at;
+  };
+  const uint32_t* status = (const uint32_t*)(b.status + p0);  // a run starts on a tile: whole words
+  uint32_t g_next = 0, f_next = n_end ? ((n_end - 1u) / FILL_LIST + 1u) * FILL_LIST : 0u;  // slots not yet listed
+  uint32_t ng = 0, gi = 0, nf = 0, fi = 0;
+  for (;;) {  // block-uniform
+    if (gi == ng) {
+      gi = ng = 0;
+      while (g_next < n_keep) {
+        const uint32_t s0 = g_next + 8u * tid;
+        const uint32_t w0 = s0 < n_keep ? status[s0 / 4] : 0u, w1 = s0 + 4 < n_keep ? status[s0 / 4 + 1] : 0u;
+        const uint32_t f = idle4(w0, s0, 0u, n_keep, false) | (idle4(w1, s0 + 4, 0u, n_keep, false) << 4);
+        uint32_t tot;
+        uint32_t at = ng + scan((uint32_t)__popc(f), tot);
+        if (ng + tot > GAP_LIST) break;  // these with the next list
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j)
+          if (f & (1u << j)) s_gap[at++] = s0 + j;
+        ng += tot;
+        g_next += GAP_LIST;
+      }
+    }
+    while (fi == nf && f_next > n_keep) {
+      f_next -= FILL_LIST;
+      const uint32_t s0 = f_next + 4u * tid;
+      const uint32_t f = idle4(s0 < n_end ? status[s0 / 4] : 0u, s0, n_keep, n_end, true);
+      uint32_t tot;
+      uint32_t at = scan((uint32_t)__popc(f), tot);
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j)
+        if (f & (1u << j)) s_fill[tot - 1u - at++] = s0 + j;
+      nf = tot;
+      fi = 0;
+    }
+    if (gi == ng || fi == nf) return;
+    __syncthreads();  // the lists are written
+    const uint32_t m = ng - gi < nf - fi ? ng - gi : nf - fi;
+    for (uint32_t k = tid; k < m; k += REMOVE_THREADS) move_particle(b, n_var, p0 + s_gap[gi + k], p0 + s_fill[fi + k]);
+    gi += m;
+    fi += m;
+  }
+}
 
-// ------------------------------------------------------------------ removal
-// Over the tiles of [0, n_end) of every compacting run (the removal layout
-// rm_tile_off, written by the bookkeeping): gaps are the non-Idle slots below
-// n_keep (ascending); fillers the Idle slots in [n_keep, n_end) (descending),
-// the step's newborns among them.  The i-th gap receives the i-th filler.
+// A tile's gaps (low 32 bits) and fillers (high) over the tiles of the removal
+// layout (rm_tile_off, written by the bookkeeping); the grid's last block
+// turns them into sums before each tile, tile_pre[0..T].  The counts cross
+// blocks, so they are stored and read at device scope.
 __global__ void __launch_bounds__(BLOCK) k_gap_count(BatchDev b) {
-  __shared__ uint32_t s_g[WAVES], s_f[WAVES];
+  __shared__ unsigned long long s_c[WAVES];
+  __shared__ uint32_t s_last;
   const uint32_t* off = b.rm_tile_off;
   const uint32_t T = off[b.R];
+  const uint32_t nb = T < gridDim.x ? T : gridDim.x;  // blocks with a tile
+  if (blockIdx.x >= nb) return;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   for (uint32_t t = blockIdx.x; t < T; t += gridDim.x) {
     const uint32_t r = find_run(off, b.R, t);
     const RunState* rs = b.rs + r;
-    const RunDev& rd = b.runs[r];
-    const uint32_t slot0 = (t - off[r]) * TILE;
+    const uint32_t s0 = (t - off[r]) * TILE + 4u * tid;
     const uint32_t n_end = rs->n_end, n_keep = rs->n_keep;
+    const uint32_t w = s0 < n_end ? *(const uint32_t*)(b.status + b.runs[r].p_off + s0) : 0u;
     uint32_t ng = 0, nf = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < PPT; ++k) {
-      const uint32_t s = slot0 + k * BLOCK + tid;
-      if (s < n_end) {
-        const bool live = b.status[rd.p_off + s] == IDLE;
-        ng += (s < n_keep && !live) ? 1u : 0u;
-        nf += (s >= n_keep && live) ? 1u : 0u;
-      }
+    for (uint32_t j = 0; j < 4; ++j) {
+      const bool live = ((w >> (8 * j)) & 0xFFu) == IDLE;
+      const uint32_t s = s0 + j;
+      ng += (s < n_keep && !live) ? 1u : 0u;
+      nf += (s >= n_keep && s < n_end && live) ? 1u : 0u;
     }
     ng = wave_sum(ng);
     nf = wave_sum(nf);
-    if (lane == 0) {
-      s_g[wave] = ng;
-      s_f[wave] = nf;
-    }
+    if (lane == 0) s_c[wave] = (unsigned long long)ng | ((unsigned long long)nf << 32);
     __syncthreads();
-    if (tid == 0) {
-      uint32_t a = 0, c = 0;
-      for (uint32_t wv = 0; wv < WAVES; ++wv) {
-        a += s_g[wv];
-        c += s_f[wv];
-      }
-      b.tile_gap[t] = a;
-      b.tile_fill[t] = c;
-    }
+    if (tid == 0)
+      __hip_atomic_store(b.tile_cnt + t, s_c[0] + s_c[1] + s_c[2] + s_c[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
   }
-}
-
-__global__ void __launch_bounds__(SCAN_THREADS) k_gap_scan(BatchDev b) {
-  const uint32_t r = blockIdx.x;
-  RunState* rs = b.rs + r;
-  if (rs->compact != 1u) return;
-  const uint32_t t0 = b.rm_tile_off[r];
-  const uint32_t nt = b.rm_tile_off[r + 1] - t0;
-  const uint32_t g = block_scan(b.tile_gap + t0, b.tile_gap_off + t0, nt, false);
-  const uint32_t f = block_scan(b.tile_fill + t0, b.tile_fill_off + t0, nt, true);
-  // gaps and fillers are equinumerous when the inactive count is right; if
-  // not, fill only as many gaps as there are listed fillers
-  if (threadIdx.x == 0) rs->gap_total = g < f ? g : f;
+  static_assert(WAVES == 4 && TILE == 4 * BLOCK, "four waves, four slots per thread");
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  uint32_t* ticket = b.ticket + (1u + RESOLVE_TICKETS) * TICKET_STRIDE;
+  if (tid == 0) s_last = atomicAdd(ticket, 1u) == nb - 1u ? 1u : 0u;
+  __syncthreads();
+  if (!s_last) return;
+  if (tid == 0) *ticket = 0u;
+  // sums before each tile: RB consecutive tiles per thread and round
+  constexpr uint32_t RB = 16;
+  unsigned long long carry = 0;
+  for (uint32_t base = 0; base < T; base += RB * BLOCK) {
+    unsigned long long v[RB], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < RB; ++j) {
+      const uint32_t t = base + tid * RB + j;
+      v[j] = t < T ? __hip_atomic_load(b.tile_cnt + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < RB; ++j) sum += v[j];
+    unsigned long long inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned long long x = __shfl_up(inc, d, 64);
+      if (lane >= (uint32_t)d) inc += x;
+    }
+    __syncthreads();  // earlier readers of s_c are done
+    if (lane == 63) s_c[wave] = inc;
+    __syncthreads();
+    unsigned long long run = carry + inc - sum;
+    for (uint32_t k = 0; k < wave; ++k) run += s_c[k];
+#pragma unroll
+    for (uint32_t j = 0; j < RB; ++j) {
+      const uint32_t t = base + tid * RB + j;
+      if (t < T) b.tile_pre[t] = run;
+      run += v[j];
+    }
+    carry += s_c[0] + s_c[1] + s_c[2] + s_c[3];
+  }
+  if (tid == 0) b.tile_pre[T] = carry;
 }
 
 // rank of this thread's flagged slots among the flagged slots of the tile,
@@ -197,71 +253,68 @@ __device__ __forceinline__ uint32_t tile_ranks(const bool (&f)[PPT], uint32_t (&
   return before;
 }
 
-__global__ void __launch_bounds__(BLOCK) k_gap_list(BatchDev b) {
-  __shared__ uint32_t s_cnt[PPT][WAVES];
-  const uint32_t* off = b.rm_tile_off;
-  const uint32_t T = off[b.R];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  for (uint32_t t = blockIdx.x; t < T; t += gridDim.x) {
-    if (b.tile_fill[t] == 0) continue;
-    const uint32_t r = find_run(off, b.R, t);
-    const RunState* rs = b.rs + r;
-    const RunDev& rd = b.runs[r];
-    const uint32_t slot0 = (t - off[r]) * TILE;
-    const uint32_t n_end = rs->n_end, n_keep = rs->n_keep;
-    bool f[PPT];
-    uint32_t rank[PPT];
-#pragma unroll
-    for (uint32_t k = 0; k < PPT; ++k) {
-      const uint32_t s = slot0 + k * BLOCK + tid;
-      f[k] = s < n_end && s >= n_keep && b.status[rd.p_off + s] == IDLE;
-    }
-    const uint32_t tot = tile_ranks(f, rank, s_cnt, lane, wave);
-    const uint32_t fo = b.tile_fill_off[t];
-#pragma unroll
-    for (uint32_t k = 0; k < PPT; ++k)
-      if (f[k]) b.fill_src[rd.p_off + fo + (tot - 1u - rank[k])] = slot0 + k * BLOCK + tid;
-  }
-}
-
+// Fills the gaps of a tile: its gaps' ranks [go, go + ng) in the run name the
+// fillers of descending rank [go, go + ng), which sit in one or a few
+// consecutive tiles; the block lists those in LDS, then moves them.
 __global__ void __launch_bounds__(BLOCK) k_gap_fill(BatchDev b, uint32_t n_var) {
   __shared__ uint32_t s_cnt[PPT][WAVES];
+  __shared__ uint32_t s_src[TILE];
   const uint32_t* off = b.rm_tile_off;
   const uint32_t T = off[b.R];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   for (uint32_t t = blockIdx.x; t < T; t += gridDim.x) {
-    if (b.tile_gap[t] == 0) continue;
+    const uint32_t ng = (uint32_t)b.tile_pre[t + 1] - (uint32_t)b.tile_pre[t];
+    if (ng == 0) continue;
     const uint32_t r = find_run(off, b.R, t);
     const RunState* rs = b.rs + r;
-    const RunDev& rd = b.runs[r];
-    const uint32_t slot0 = (t - off[r]) * TILE;
-    const uint32_t n_keep = rs->n_keep;
+    const uint64_t p0 = b.runs[r].p_off;
+    const uint32_t t0 = off[r], t1 = off[r + 1];
+    const unsigned long long pre0 = b.tile_pre[t0];
+    const uint32_t f0 = (uint32_t)(pre0 >> 32);
+    const uint32_t F = (uint32_t)(b.tile_pre[t1] >> 32) - f0;  // the run's fillers
+    const uint32_t go = (uint32_t)b.tile_pre[t] - (uint32_t)pre0;
+    const uint32_t n_end = rs->n_end, n_keep = rs->n_keep;
+    // ascending ranks [qa, qb) of the fillers wanted (fewer than ng when they run out)
+    const uint32_t qb = F > go ? F - go : 0u, qa = F > go + ng ? F - go - ng : 0u;
+    if (qa >= qb) continue;
+    // the last tile whose fillers start at or before rank qa
+    uint32_t lo = t0, hi = t1;
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if ((uint32_t)(b.tile_pre[mid] >> 32) - f0 <= qa) lo = mid; else hi = mid;
+    }
+    for (uint32_t ft = lo; ft < t1; ++ft) {
+      const uint32_t fb = (uint32_t)(b.tile_pre[ft] >> 32) - f0;  // rank of the tile's first filler
+      if (fb >= qb) break;
+      bool f[PPT];
+      uint32_t rank[PPT];
+#pragma unroll
+      for (uint32_t k = 0; k < PPT; ++k) {
+        const uint32_t s = (ft - t0) * TILE + k * BLOCK + tid;
+        f[k] = s < n_end && s >= n_keep && b.status[p0 + s] == IDLE;
+      }
+      tile_ranks(f, rank, s_cnt, lane, wave);
+#pragma unroll
+      for (uint32_t k = 0; k < PPT; ++k) {
+        const uint32_t q = fb + rank[k];
+        if (f[k] && q >= qa && q < qb) s_src[q - qa] = (ft - t0) * TILE + k * BLOCK + tid;
+      }
+    }
+    const uint32_t slot0 = (t - t0) * TILE;
     bool f[PPT];
     uint32_t rank[PPT];
 #pragma unroll
     for (uint32_t k = 0; k < PPT; ++k) {
       const uint32_t s = slot0 + k * BLOCK + tid;
-      f[k] = s < n_keep && b.status[rd.p_off + s] != IDLE;
+      f[k] = s < n_keep && b.status[p0 + s] != IDLE;
     }
-    tile_ranks(f, rank, s_cnt, lane, wave);
-    const uint32_t go = b.tile_gap_off[t];
-    const uint32_t n_fill = rs->gap_total;
-    const uint32_t n_end = rs->n_end;
+    tile_ranks(f, rank, s_cnt, lane, wave);  // its barriers also put s_src before its readers
 #pragma unroll
     for (uint32_t k = 0; k < PPT; ++k) {
-      if (!f[k] || go + rank[k] >= n_fill) continue;
-      const uint32_t src_slot = b.fill_src[rd.p_off + go + rank[k]];
-      if (src_slot >= n_end) continue;
-      const uint64_t dst = rd.p_off + slot0 + k * BLOCK + tid;
-      const uint64_t src = rd.p_off + src_slot;
-      b.pos[dst] = b.pos[src];
-      b.status[dst] = IDLE;
-      b.age_hyd[dst] = b.age_hyd[src];
-      b.age_div[dst] = b.age_div[src];
-      b.clk_hyd[dst] = b.clk_hyd[src];
-      b.clk_div[dst] = b.clk_div[src];
-      for (uint32_t v = 0; v < n_var; ++v) b.state[(uint64_t)v * b.P + dst] = b.state[(uint64_t)v * b.P + src];
+      if (!f[k] || rank[k] >= qb - qa) continue;
+      move_particle(b, n_var, p0 + slot0 + k * BLOCK + tid, p0 + s_src[qb - 1u - rank[k] - qa]);
     }
+    __syncthreads();  // s_src is read before the next tile's list
   }
 }
 
@@ -325,10 +378,12 @@ const ModelOps* builtin_model_ops(int model_id) {
   return &ops[model_id];
 }
 
-void launch_removal(const BatchDev& b, uint32_t n_var, int grid, hipStream_t s) {
+void launch_removal(const BatchDev& b, uint32_t n_var, int grid, uint32_t max_tiles, hipStream_t s) {
+  if (max_tiles <= REMOVE_RUN_TILES) {
+    hipLaunchKernelGGL(k_remove_runs, dim3(b.R), dim3(REMOVE_THREADS), 0, s, b, n_var);
+    return;
+  }
   hipLaunchKernelGGL(k_gap_count, dim3(grid), dim3(BLOCK), 0, s, b);
-  hipLaunchKernelGGL(k_gap_scan, dim3(b.R), dim3(SCAN_THREADS), 0, s, b);
-  hipLaunchKernelGGL(k_gap_list, dim3(grid), dim3(BLOCK), 0, s, b);
   hipLaunchKernelGGL(k_gap_fill, dim3(grid), dim3(BLOCK), 0, s, b, n_var);
 }
 

@@ -44,7 +44,8 @@ struct ModelOps {
 };
 const ModelOps* builtin_model_ops(int model_id);
 
-void launch_removal(const BatchDev& b, uint32_t n_var, int grid, hipStream_t s);
+// max_tiles: slot capacity of the largest run on the device, in tiles
+void launch_removal(const BatchDev& b, uint32_t n_var, int grid, uint32_t max_tiles, hipStream_t s);
 void launch_layout(const BatchDev& b, hipStream_t s);
 void launch_repartition(const BatchDev& b, uint32_t run, uint32_t n_c, unsigned long long* hist, hipStream_t s);
 void launch_clear_u64(unsigned long long* p, uint64_t n, hipStream_t s);

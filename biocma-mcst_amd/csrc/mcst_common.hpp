@@ -27,6 +27,7 @@ constexpr uint32_t WAVES = BLOCK / 64;
 constexpr uint32_t RESOLVE_GROUP_MAX = 64;  // sub-chunks per group of the resolve kernel: 32 or 64 (at most 256)
 constexpr uint32_t RESOLVE_TICKETS = 64;    // sub-counters of the resolve kernel's done-count
 constexpr uint32_t TICKET_STRIDE = 32;      // words between two of those counters (a line each)
+constexpr uint32_t REMOVE_RUN_TILES = 512;  // largest capacity at which one block removes a run's inactive slots
 constexpr uint32_t DIV_STAGE = 16;          // division requests per sub-chunk divided in the particle pass
 constexpr int MAX_PARAMS = 16;
 constexpr int MAX_VAR = 16;
@@ -173,7 +174,6 @@ struct RunState {
   uint32_t births;          // newborns of the last step
   uint32_t tile_begin;      // first global tile of the run in the current layout
   uint32_t n_tiles;         // tiles of the run in the current layout
-  uint32_t gap_total;
   uint32_t active;          // 1 while step < step_target
   // age clocks: the steps so far in which the run's Idle particles aged
   // (division age: steps with the model stage; hydraulic age: steps with the
@@ -225,14 +225,12 @@ struct BatchDev {
   uint32_t* div_l1;
   uint32_t* div_l2;
   uint32_t* div_l3;
-  uint32_t* ticket;         // [1 + RESOLVE_TICKETS][TICKET_STRIDE] resolve blocks that are done (the last keeps the books)
+  uint32_t* ticket;         // [2 + RESOLVE_TICKETS][TICKET_STRIDE] resolve blocks that are done (the last keeps the books);
+                            // the last row: the removal's counting blocks
   uint32_t* rm_tile_off;    // [R+1] removal layout: first global tile of each run's [0, n_end)
   // per-tile bookkeeping of the removal
-  uint32_t* tile_gap;
-  uint32_t* tile_fill;
-  uint32_t* tile_gap_off;
-  uint32_t* tile_fill_off;
-  uint32_t* fill_src;       // [P] scratch list of filler slots during removal
+  unsigned long long* tile_cnt;  // [T_max] gaps (low 32 bits) and fillers (high) of each tile
+  unsigned long long* tile_pre;  // [T_max+1] their sums before each tile
   uint32_t* tile_off;       // [R+1] first global tile of each run in the current layout
   // lists of the particle pass, one segment of TILE/nsub entries per sub-chunk
   uint32_t* move_rec;       // [T_max*TILE] particles leaving their compartment, one entry each

@@ -280,7 +280,7 @@ int mcst_engine_synchronize(mcst_engine* e);
 /* Take n steps, as mcst_engine_step, timed with HIP events on the engine
  * stream: total ms and the mean duration of each step kernel, in the order
  * transport (with the tile layout), particle pass, mover and division
- * resolution (with the bookkeeping), removal (4 kernels together, skipped
+ * resolution (with the bookkeeping), removal (one or two kernels, skipped
  * when no particle can become inactive) -> per_kernel_ms[4]. */
 int mcst_engine_profile(mcst_engine* e, uint32_t n_steps, double* total_ms, double* per_kernel_ms);
 /* Autotuner of the particle pass (no counterpart in the reference; the
