@@ -117,7 +117,9 @@ struct RunDev {
   double params[MAX_PARAMS];
   double* C[2];             // [n_s][n_c] concentrations, ping-pong by step parity
   double* m;                // [n_s][n_c] liquid mass
-  double* S;                // [n_s][n_c] particle sources of the current step
+  double* S;                // [n_s][n_c] particle sources of the last step, as the host may read them
+  double* Sp;               // [copies][n_s][n_c] the pass adds to these; zero but between a pass and
+                            // its resolve kernel
   const double* F;          // [n_s][n_c] constant feed sources
   const double* sink;       // [n_c]      outlet flow per compartment
   const double* kla;        // [n_s][n_c] gas-liquid transfer coefficient (null: no transfer)
@@ -258,23 +260,24 @@ struct BatchDev {
   uint32_t tile_group;      // particle pass: consecutive tiles per block turn (0: one range per block)
   uint32_t acc_w;           // particle pass: compartments per LDS contribution window (PRIV)
   uint32_t stages;
-  // contribution rows (one live run whose whole [n_s][n_c] accumulator fits
-  // LDS): block k of the particle pass stores its accumulator at
-  // part[k * part_w] (part_rows blocks, part_w = n_s * n_c) and the resolve
-  // kernel sums the rows; null: the blocks add their accumulators to S with
-  // atomics
-  double* part;
-  uint32_t part_rows;
-  uint32_t part_w;
-  uint32_t part_run;        // the run the rows belong to
+  // copies of each run's contribution accumulator in use (1 or run_copies): block
+  // k of the particle pass adds to copy k % n_copies, and the resolve kernel
+  // sums the copies
+  uint32_t n_copies;
 };
 
-// Compartments per block of the row sum: (NS species x PART_CPB values) per
-// thread and row.
-template <int NS>
-constexpr uint32_t part_cpb() {
-  return NS >= 16 ? 1u : 16u / (uint32_t)NS;
-}
+// A pass ends with every block adding its LDS accumulator to the run's, a
+// line's adds one after another; blocks are dealt to the XCDs in turn, so with
+// 8 copies an XCD's blocks queue on their own lines only.  338 blocks of a
+// 345 679-particle pass took 16.2 us with one copy, 13.9 with 4 and 12.2 with 8,
+// 512 blocks of the 1e7-particle pass 126, 123 and 123 (the resolve kernel 11.0,
+// 10.8 and 13.9 us: 8 copies of 2 species spill).  Copies cost their sum and their clearing, so
+// they are kept to batches of at most S_COPY_ENTRIES values in all (the
+// blocks of a larger batch or network meet on fewer of its lines).
+constexpr uint32_t S_COPIES = 8, S_COPY_ENTRIES = 16384;
+// ... of a model with ns species: fewer where the thread that sums a
+// compartment's copies would hold more than 16 of them in registers
+constexpr uint32_t run_copies(int ns) { return ns == 1 ? S_COPIES : ns == 2 ? S_COPIES / 2 : S_COPIES / 4; }
 
 // Age of a slot from its base age, its origin on the age clock and the
 // clock (the expression the host's conversion uses too).

@@ -89,7 +89,7 @@ constexpr uint32_t SCAN_WAVES = SCAN_THREADS / 64;
 // compartment of every active run, one thread each, all species at once (the
 // flow matrix entries are read once for all of them); also refreshes the
 // per-compartment record {M::record(C), p_move, q_exit} the particle pass
-// gathers, and clears S.  The extra last block lays out the step's tiles
+// gathers.  The extra last block lays out the step's tiles
 // (layout_pass), which needs only the counts of the previous step.
 template <uint32_t NT>
 __device__ void layout_pass(const BatchDev& b);
@@ -99,13 +99,13 @@ __device__ void layout_pass(const BatchDev& b);
 // are all in flight together (a column holds the degree plus the diagonal,
 // rarely more than 8); the sums still run in entry order.
 template <int NS>
-__device__ __forceinline__ void column_inflow(const uint32_t* __restrict__ col_ptr, const uint32_t* __restrict__ src,
-                                              const double* __restrict__ val, const double* c, uint32_t n_c,
+__device__ __forceinline__ void column_inflow(const GLOBAL_AS uint32_t* col_ptr, const GLOBAL_AS uint32_t* src,
+                                              const GLOBAL_AS double* val, const GLOBAL_AS double* c, uint32_t n_c,
                                               uint32_t j, double (&acc)[NS]) {
 #pragma unroll
   for (int s = 0; s < NS; ++s) acc[s] = 0.0;
   const uint32_t e0 = col_ptr[j], e1 = col_ptr[j + 1];
-  constexpr uint32_t EG = NS >= 4 ? 4u : 8u;  // entries in flight: fewer for many species (registers)
+  constexpr uint32_t EG = NS >= 2 ? 4u : 8u;  // entries in flight: fewer for many species (registers)
   for (uint32_t e = e0; e < e1; e += EG) {
     uint32_t i[EG];
     double v[EG], cv[EG][NS];
@@ -130,192 +130,176 @@ __device__ __forceinline__ void column_inflow(const uint32_t* __restrict__ col_p
 // The transport of batch compartment g for the step `ahead` steps after its
 // run's current one (0: the step about to run; 1: the next one, computed
 // during this step's resolve kernel).  It reads C and the contributions of
-// the last pass, from S (s_in null; S is then cleared) or from s_in (the
-// compartment's NS summed contribution rows), and writes the other C buffer,
-// m and the record table of its step's parity; the resolve kernel reads none
-// of these but the other record table.
-template <class M>
-__device__ void transport_one(const BatchDev& b, uint32_t g, uint32_t ahead, const double* s_in) {
+// the last pass, from S or (TAKE > 0) from the TAKE accumulators the pass has
+// just filled, which it clears, and writes the other C buffer, m and the record
+// table of its step's parity; the resolve kernel reads none of these but the
+// other record table.  The copies' loads are issued first and summed where the
+// sum is used, behind the flow columns' chain of loads (a lane per copy and a
+// sum by shuffles before that chain cost the resolve kernel 2 us).  TAKE
+// without a next step of this call or of the run (`ahead` 0, or the run's step
+// target): the sums go to S, so that S holds the step's contributions
+// whenever the host can read it.
+//
+// Every load comes before the first store (the arrays may alias as far as the
+// compiler knows: a store in between made it read the run's and the flowmap's
+// fields again, a round trip each).
+template <class M, int TAKE>
+__device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* __restrict__ runs,
+                                              const MapDev* __restrict__ maps, uint32_t g, uint32_t ahead) {
   constexpr int NS = M::NS;
-  {
-    const uint32_t r = find_run(b.comp_off, b.R, g);
-    const RunDev& rd = b.runs[r];
-    const RunState* rs = b.rs + r;
-    // the step being prepared; the run's activity is recomputed here rather
-    // than read from the layout, which other blocks write concurrently
-    const uint32_t step = rs->step + ahead;
-    if (step >= rd.step_target) return;
-    const uint32_t j = g - b.comp_off[r];
-    const uint32_t n_c = rd.n_c;
-    const MapDev& mp = b.maps[rd.map_base + (step / rd.steps_per_map) % rd.n_maps];
-    constexpr int NR = record_terms<M>();
-    double* rec = rd.rec + ((size_t)(step & 1u) * n_c + j) * rd.rec_w;
-    rec[NR] = mp.p_move[j];
-    double qx = mp.q_exit[j];
-    if (rd.n_vf && rd.vx_slot[j] >= 0) qx = rd.vf_q[rd.n_vf + (uint32_t)rd.vx_slot[j]];
-    rec[NR + 1] = qx;
-    const double* c = rd.C[step & 1u];
-    double* Cn = rd.C[(step + 1u) & 1u];
-    double cn[NS];
+  constexpr int NR = record_terms<M>();
+  constexpr uint32_t KM = TAKE ? (uint32_t)TAKE : 1u;
+  const uint32_t r = find_run(b.comp_off, b.R, g);
+  const RunDev& rd = runs[r];
+  // the step being prepared; the run's activity is recomputed here rather
+  // than read from the layout, which other blocks write concurrently
+  const uint32_t step = b.rs[r].step + ahead;
+  if (step - ahead >= rd.step_target) return;  // the run did not take (or does not take) this step
+  const uint32_t j = g - b.comp_off[r];
+  const uint32_t n_c = rd.n_c;
+  // the contributions of the last pass
+  double sp[KM][NS];
+  GLOBAL_AS double* const from = gp(TAKE ? rd.Sp : rd.S) + j;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) cn[s] = c[(size_t)s * n_c + j];
-    if (b.stages & STAGE_TRANSPORT) {
-      double acc[NS];
-      column_inflow<NS>(mp.col_ptr, mp.src, mp.val, c, n_c, j, acc);
-      double sink = rd.sink[j];
-      const double inv_v = mp.inv_v[j];
-      const bool gas = rd.Cg[0] != nullptr;
-      double fv[NS], fvg[NS];  // time-dependent feeds of this compartment, in feed order
-      double sink_g = gas ? rd.sink_g[j] : 0.0;
+  for (uint32_t k = 0; k < KM; ++k)
 #pragma unroll
-      for (int s = 0; s < NS; ++s) fv[s] = fvg[s] = 0.0;
-      if (rd.n_vf) {
-        for (uint32_t q = rd.vf_sink_ptr[j]; q < rd.vf_sink_ptr[j + 1]; ++q) {
-          const uint32_t k = rd.vf_sink_k[q];
-          if (k & VF_GAS)
-            sink_g = sink_g + rd.vf_q[k & ~VF_GAS];
-          else
-            sink = sink + rd.vf_q[k];
-        }
-        for (uint32_t q = rd.vf_src_ptr[j]; q < rd.vf_src_ptr[j + 1]; ++q) {
-          const double add = rd.vf_q[rd.vf_src_k[q]] * rd.vf_src_c[q];
-          const uint32_t sp = rd.vf_src_s[q];
+    for (int s = 0; s < NS; ++s) sp[k][s] = from[((size_t)k * NS + s) * n_c];
+  auto source = [&](int s) -> double {
+    double t = sp[0][s];
 #pragma unroll
-          for (int s = 0; s < NS; ++s) {
-            if ((uint32_t)s == sp) fv[s] += add;
-            if (((uint32_t)s | VF_GAS) == sp) fvg[s] += add;
-          }
-        }
+    for (uint32_t k = 1; k < KM; ++k) t += sp[k][s];
+    return t;
+  };
+  auto clear = [&]() {
+#pragma unroll
+    for (uint32_t k = 0; k < KM; ++k)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) from[((size_t)k * NS + s) * n_c] = 0.0;
+  };
+  if (TAKE && (!ahead || step >= rd.step_target)) {
+    GLOBAL_AS double* const S = gp(rd.S) + j;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) S[(size_t)s * n_c] = source(s);
+    clear();
+    return;
+  }
+  const MapDev& mp = maps[rd.map_base + (step / rd.steps_per_map) % rd.n_maps];
+  const double p_move = gp(mp.p_move)[j];
+  double qx = gp(mp.q_exit)[j];
+  if (rd.n_vf && rd.vx_slot[j] >= 0) qx = rd.vf_q[rd.n_vf + (uint32_t)rd.vx_slot[j]];
+  const GLOBAL_AS double* c = gp(rd.C[step & 1u]);
+  const bool gas = rd.Cg[0] != nullptr;
+  double cn[NS], mn[NS];  // new concentrations and masses
+#pragma unroll
+  for (int s = 0; s < NS; ++s) cn[s] = c[(size_t)s * n_c + j];
+  if (b.stages & STAGE_TRANSPORT) {
+    double acc[NS];
+    column_inflow<NS>(gp(mp.col_ptr), gp(mp.src), gp(mp.val), c, n_c, j, acc);
+    double sink = gp(rd.sink)[j];
+    const double inv_v = gp(mp.inv_v)[j];
+    double fv[NS], fvg[NS];  // time-dependent feeds of this compartment, in feed order
+    double sink_g = gas ? gp(rd.sink_g)[j] : 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) fv[s] = fvg[s] = 0.0;
+    if (rd.n_vf) {
+      for (uint32_t q = rd.vf_sink_ptr[j]; q < rd.vf_sink_ptr[j + 1]; ++q) {
+        const uint32_t k = rd.vf_sink_k[q];
+        if (k & VF_GAS)
+          sink_g = sink_g + rd.vf_q[k & ~VF_GAS];
+        else
+          sink = sink + rd.vf_q[k];
       }
-      if (gas) {
-        // two-phase step (SimulationUnit::ode_step, simulation.model.cpp:131-150):
-        // mtr = kla*(H*C_gas - C)*V from the old concentrations, the gas
-        // step with -mtr and the liquid step with +mtr (performStepGL,
-        // implScalar.cpp:228-248), then clearNegs on the liquid
-        // (implScalar.cpp:266-297): a value in (-1e-4*5e-3, 0) becomes 0
-        const double* cg = rd.Cg[step & 1u];
-        double* Cgn = rd.Cg[(step + 1u) & 1u];
-        double accg[NS];
-        column_inflow<NS>(mp.g_col_ptr, mp.g_src, mp.g_val, cg, n_c, j, accg);
-        const double inv_vg = mp.g_inv_v[j];
-        const double tol = 1e-4 * 5e-3;
+      for (uint32_t q = rd.vf_src_ptr[j]; q < rd.vf_src_ptr[j + 1]; ++q) {
+        const double add = rd.vf_q[rd.vf_src_k[q]] * rd.vf_src_c[q];
+        const uint32_t sp = rd.vf_src_s[q];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-          const size_t o = (size_t)s * n_c + j;
-          const double cgs = cg[o];
-          const double mtr = (mp.g_kla[o] * ((cgs * rd.henry[s]) - cn[s])) * mp.vol[j];
-          const double dg = ((accg[s] - cgs * sink_g) + (rd.Fg[o] + fvg[s])) - mtr;
-          const double mgo = rd.mg[o] + rd.dt * dg;
-          rd.mg[o] = mgo;
-          Cgn[o] = mgo * inv_vg;
-          const double sv = s_in ? s_in[s] : rd.S[o];  // the contributions of the last pass
-          const double dl = ((acc[s] - cn[s] * sink) + (sv + (rd.F[o] + fv[s]))) + mtr;
-          const double mm = rd.m[o] + rd.dt * dl;
-          rd.m[o] = mm;
-          double cl = mm * inv_v;
-          if (cl < 0.0 && fabs(cl) < tol) cl = 0.0;
-          cn[s] = cl;
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const size_t o = (size_t)s * n_c + j;
-          const double sv = s_in ? s_in[s] : rd.S[o];  // the contributions of the last pass
-          double dmdt = (acc[s] - cn[s] * sink) + (sv + (rd.F[o] + fv[s]));
-          // gas-liquid transfer from a fixed gas phase: kla*(C* - C)*V
-          if (rd.kla) dmdt = dmdt + (rd.kla[o] * (rd.cstar[o] - cn[s])) * mp.vol[j];
-          const double mm = rd.m[o] + rd.dt * dmdt;
-          rd.m[o] = mm;
-          cn[s] = mm * inv_v;
+          if ((uint32_t)s == sp) fv[s] += add;
+          if (((uint32_t)s | VF_GAS) == sp) fvg[s] += add;
         }
       }
     }
-    double rt[NR];
-    M::record(rd.params, cn, rt);
+    if (gas) {
+      // two-phase step (SimulationUnit::ode_step, simulation.model.cpp:131-150):
+      // mtr = kla*(H*C_gas - C)*V from the old concentrations, the gas
+      // step with -mtr and the liquid step with +mtr (performStepGL,
+      // implScalar.cpp:228-248), then clearNegs on the liquid
+      // (implScalar.cpp:266-297): a value in (-1e-4*5e-3, 0) becomes 0
+      const GLOBAL_AS double* cg = gp(rd.Cg[step & 1u]);
+      double accg[NS];
+      column_inflow<NS>(gp(mp.g_col_ptr), gp(mp.g_src), gp(mp.g_val), cg, n_c, j, accg);
+      const double inv_vg = gp(mp.g_inv_v)[j];
+      const double tol = 1e-4 * 5e-3;
+      double cgn[NS], mgn[NS];
 #pragma unroll
-    for (int k = 0; k < NR; ++k) rec[k] = rt[k];
+      for (int s = 0; s < NS; ++s) {
+        const size_t o = (size_t)s * n_c + j;
+        const double cgs = cg[o];
+        const double mtr = (gp(mp.g_kla)[o] * ((cgs * rd.henry[s]) - cn[s])) * gp(mp.vol)[j];
+        const double dg = ((accg[s] - cgs * sink_g) + (gp(rd.Fg)[o] + fvg[s])) - mtr;
+        mgn[s] = gp(rd.mg)[o] + rd.dt * dg;
+        cgn[s] = mgn[s] * inv_vg;
+        const double dl = ((acc[s] - cn[s] * sink) + (source(s) + (gp(rd.F)[o] + fv[s]))) + mtr;
+        mn[s] = gp(rd.m)[o] + rd.dt * dl;
+        double cl = mn[s] * inv_v;
+        if (cl < 0.0 && fabs(cl) < tol) cl = 0.0;
+        cn[s] = cl;
+      }
+      GLOBAL_AS double* const Cgn = gp(rd.Cg[(step + 1u) & 1u]) + j;
+      GLOBAL_AS double* const mg_out = gp(rd.mg) + j;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const size_t o = (size_t)s * n_c + j;
-      Cn[o] = cn[s];
-      if (!s_in) rd.S[o] = 0.0;
+      for (int s = 0; s < NS; ++s) {
+        Cgn[(size_t)s * n_c] = cgn[s];
+        mg_out[(size_t)s * n_c] = mgn[s];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const size_t o = (size_t)s * n_c + j;
+        double dmdt = (acc[s] - cn[s] * sink) + (source(s) + (gp(rd.F)[o] + fv[s]));
+        // gas-liquid transfer from a fixed gas phase: kla*(C* - C)*V
+        if (rd.kla) dmdt = dmdt + (gp(rd.kla)[o] * (gp(rd.cstar)[o] - cn[s])) * gp(mp.vol)[j];
+        mn[s] = gp(rd.m)[o] + rd.dt * dmdt;
+        cn[s] = mn[s] * inv_v;
+      }
     }
   }
+  double rt[NR];
+  M::record(rd.params, cn, rt);
+  GLOBAL_AS double* const rec = gp(rd.rec) + ((size_t)(step & 1u) * n_c + j) * rd.rec_w;
+  GLOBAL_AS double* const Cn = gp(rd.C[(step + 1u) & 1u]) + j;
+  GLOBAL_AS double* const m_out = gp(rd.m) + j;
+#pragma unroll
+  for (int k = 0; k < NR; ++k) rec[k] = rt[k];
+  rec[NR] = p_move;
+  rec[NR + 1] = qx;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const size_t o = (size_t)s * n_c;
+    Cn[o] = cn[s];
+    if (b.stages & STAGE_TRANSPORT) m_out[o] = mn[s];
+  }
+  if constexpr (TAKE > 0) clear();
 }
 
-// The transport of every active run's compartments (transport_one from S),
-// by blocks `blk` of `n_blk`.
-template <class M>
-__device__ void transport_compartments(const BatchDev& b, uint32_t blk, uint32_t n_blk, uint32_t ahead) {
+// The transport (or, TAKE, what becomes of the pass's contributions) of every
+// active run's compartments, by blocks `blk` of `n_blk`.
+template <class M, int TAKE>
+__device__ void transport_compartments(const BatchDev& b, const RunDev* __restrict__ runs,
+                                       const MapDev* __restrict__ maps, uint32_t blk, uint32_t n_blk, uint32_t ahead) {
   const uint32_t total = b.n_comp_total;
   const uint32_t stride = n_blk * blockDim.x;
-  for (uint32_t g = blk * blockDim.x + threadIdx.x; g < total; g += stride) transport_one<M>(b, g, ahead, nullptr);
-}
-
-// With contribution rows: block `blk` of the resolve kernel's aux blocks sums
-// the rows of compartments [blk*CPB, (blk+1)*CPB) of the run, every species,
-// in a fixed order (each lane its rows in turn, then the wave's four lane
-// groups by a butterfly, then the waves in turn), then transports those compartments for the
-// next step with the sums (ahead) or stores the sums in S (the last step of a
-// call or of the run, so that S holds the step's contributions whenever the
-// host can read it).
-template <class M>
-__device__ void sum_rows(const BatchDev& b, uint32_t blk, bool ahead) {
-  constexpr int NS = M::NS;
-  constexpr uint32_t CPB = part_cpb<NS>();
-  constexpr uint32_t NE = (uint32_t)NS * CPB;  // 16: entries of the block, one per lane of a group of 16
-  constexpr uint32_t NWV = 256 / 64;
-  static_assert(NE <= 16, "at most 16 entries per block");
-  __shared__ double s_wsum[NWV][16];
-  __shared__ double s_sum[16];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t r = b.part_run;
-  const RunDev& rd = b.runs[r];
-  const uint32_t n_c = rd.n_c;
-  const uint32_t c0 = blk * CPB;
-  // lane group g (16 lanes) takes rows g, g + 16, ...; lane e of the group
-  // the entry e = species s, compartment c0 + k: a wave's load covers four
-  // rows, 64 contiguous bytes of each per species
-  const uint32_t e = tid & 15u, grp16 = tid >> 4;
-  const uint32_t sp = e / CPB, k = e % CPB;
-  const bool on = e < NE && c0 + k < n_c;
-  const size_t off = on ? (size_t)sp * n_c + c0 + k : 0;
-  double acc = 0.0;
-#pragma unroll 8
-  for (uint32_t row = grp16; row < b.part_rows; row += 16u)
-    if (on) acc += b.part[(size_t)row * b.part_w + off];
-  acc += __shfl_xor(acc, 16, 64);
-  acc += __shfl_xor(acc, 32, 64);
-  if (lane < 16) s_wsum[wave][lane] = acc;
-  __syncthreads();
-  if (tid < 16) {
-    double t = 0.0;
-#pragma unroll
-    for (uint32_t w = 0; w < NWV; ++w) t += s_wsum[w][tid];
-    s_sum[tid] = t;
-  }
-  __syncthreads();
-  if (tid < CPB && c0 + tid < n_c) {
-    double sv[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) sv[s] = s_sum[s * CPB + tid];
-    const uint32_t step = b.rs[r].step;  // the books advance it after every aux block is done
-    if (ahead && step + 1u < rd.step_target) {
-      transport_one<M>(b, b.comp_off[r] + c0 + tid, 1u, sv);
-    } else if (step < rd.step_target) {  // the run took this step, its last of the call or its last
-#pragma unroll
-      for (int s = 0; s < NS; ++s) rd.S[(size_t)s * n_c + c0 + tid] = sv[s];
-    }
-  }
+  for (uint32_t g = blk * blockDim.x + threadIdx.x; g < total; g += stride) transport_one<M, TAKE>(b, runs, maps, g, ahead);
 }
 
 template <class M>
-__global__ void __launch_bounds__(256) k_transport(BatchDev b) {
+__global__ void __launch_bounds__(256) k_transport(BatchDev b, const RunDev* __restrict__ runs,
+                                                  const MapDev* __restrict__ maps) {
   if (blockIdx.x == gridDim.x - 1) {
     layout_pass<256>(b);
     return;
   }
-  transport_compartments<M>(b, blockIdx.x, gridDim.x - 1, 0u);
+  transport_compartments<M, 0>(b, runs, maps, blockIdx.x, gridDim.x - 1, 0u);
 }
 
 // ------------------------------------------------------------------ particles
@@ -491,15 +475,8 @@ __global__ void __launch_bounds__(BLK)
   const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
   const uint32_t G = b.tile_group ? b.tile_group : (chunk ? chunk : 1u);
   uint32_t grp = blockIdx.x * G;
-  // contribution rows: this block's row of the pass (rows of all blocks are
-  // summed by the resolve kernel)
-  GLOBAL_AS double* const part_row =
-      (PRIV && !WIN && b.part && blockIdx.x < b.part_rows) ? gp(b.part) + (size_t)blockIdx.x * b.part_w : nullptr;
-  if (grp >= n_groups) {  // the whole block: its row holds nothing
-    if (part_row)
-      for (uint32_t i = threadIdx.x; i < b.part_w; i += BLK) part_row[i] = 0.0;
-    return;
-  }
+  if (grp >= n_groups) return;  // the whole block
+  const uint32_t copy = blockIdx.x & (b.n_copies - 1u);  // of each run's accumulator
   auto next_group = [&](uint32_t g) -> uint32_t {
     const uint32_t g0 = g - g % G;
     return (g + 1 < g0 + G) ? g + 1 : g0 + gridDim.x * G;
@@ -632,7 +609,7 @@ __global__ void __launch_bounds__(BLK)
         __syncthreads();
         flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
         acc_run = r0;
-        acc_S = gp(runs[r0].S);
+        acc_S = gp(runs[r0].Sp) + (size_t)copy * runs[r0].n_s * runs[r0].n_c;
         acc_ns = runs[r0].n_s;
         acc_nc = runs[r0].n_c;
         acc_win = acc_nc;
@@ -696,7 +673,7 @@ __global__ void __launch_bounds__(BLK)
     const double w = rd.weight;
     const uint32_t n_c = rd.n_c;
     const uint64_t seed = rd.seed;
-    GLOBAL_AS double* __restrict__ S = gp(rd.S);
+    GLOBAL_AS double* __restrict__ S = gp(rd.Sp) + (size_t)copy * NS * n_c;  // contributions outside LDS
     const bool to_lds = PRIV && r == acc_run;
     double p[NP];
 #pragma unroll
@@ -939,11 +916,7 @@ __global__ void __launch_bounds__(BLK)
   }
   if (PRIV) {
     __syncthreads();
-    if (part_row) {  // the accumulator of the one run, every entry
-      for (uint32_t i = tid; i < b.part_w; i += BLK) part_row[i] = s_acc[i];
-    } else {
-      flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
-    }
+    flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
   }
   flush_counts();
 #pragma unroll
@@ -1152,16 +1125,17 @@ __device__ __forceinline__ uint32_t request_prefix(const BatchDev& b, uint32_t s
 }
 
 // The resolve kernel.  The grid's first tr_blocks blocks (dispatched first:
-// their chain is the shorter) are aux blocks.  With `ahead` they transport
-// the liquid (and gas) for the next step meanwhile: the two touch disjoint
-// data (the records of the two steps are separate tables, the concentrations
-// are double-buffered), and the block that keeps the books also lays out the
-// next step's tiles, so the next step starts with its particle pass.  With
-// contribution rows (ROWS: the variant launched when b.part is set; the
-// other one keeps no code of it, which would cost it registers) they first
-// sum the pass's rows, for that transport or, without `ahead`, into S.
-template <class M, bool ROWS>
-__global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __restrict__ runs,
+// their chain is the shorter) are aux blocks: they take the pass's
+// contributions and, with `ahead`, transport the liquid
+// (and gas) for the next step meanwhile: the two touch disjoint data (the
+// records of the two steps are separate tables, the concentrations are
+// double-buffered), and the block that keeps the books also lays out the next
+// step's tiles, so the next step starts with its particle pass.  K: copies of
+// the accumulators (a variant each, as the copies' registers cost the others
+// occupancy: one copy's taking turns of 8 copies' code made the resolve kernel
+// of a 40-run batch 24 us instead of 20).
+template <class M, int K>
+__global__ void __launch_bounds__(256, M::NV <= 8 ? 4 : 1) k_resolve(BatchDev b, const RunDev* __restrict__ runs,
                                                  const MapDev* __restrict__ maps,
                                                  const uint32_t* __restrict__ tile_off, uint32_t tr_blocks,
                                                  uint32_t ahead) {
@@ -1197,10 +1171,7 @@ __global__ void __launch_bounds__(256) k_resolve(BatchDev b, const RunDev* __res
   uint32_t ev_run = 0, ev_moves = 0, ev_req = 0;  // movers and requests of the block's groups (thread 0)
   const bool leave_stage = (b.stages & STAGE_LEAVE) != 0;
   if (tr_block) {
-    if constexpr (ROWS)
-      sum_rows<M>(b, blockIdx.x, ahead != 0);
-    else
-      transport_compartments<M>(b, blockIdx.x, tr_blocks, 1u);
+    transport_compartments<M, K>(b, runs, maps, blockIdx.x, tr_blocks, ahead);
   }
   for (uint32_t grp = rb; !tr_block && grp < n_groups; grp += n_res) {
     const uint32_t sc0 = grp * GS;
@@ -1648,20 +1619,20 @@ static void launch_t(const BatchDev& b, const ParticleLaunch& L, hipStream_t s) 
 
 template <class M>
 void transport_t(const BatchDev& b, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(k_transport<M>, dim3(grid), dim3(256), 0, s, b);
+  hipLaunchKernelGGL(k_transport<M>, dim3(grid), dim3(256), 0, s, b, b.runs, b.maps);
 }
 template <class M>
 void resolve_t(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s) {
-  if (b.part)
-    hipLaunchKernelGGL((k_resolve<M, true>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
+  if (b.n_copies == 1)
+    hipLaunchKernelGGL((k_resolve<M, 1>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
                        (const uint32_t*)b.tile_off, aux, ahead ? 1u : 0u);
   else
-    hipLaunchKernelGGL((k_resolve<M, false>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
+    hipLaunchKernelGGL((k_resolve<M, (int)run_copies(M::NS)>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
                        (const uint32_t*)b.tile_off, aux, ahead ? 1u : 0u);
 }
 template <class M>
-const void* resolve_kernel_t() {
-  return (const void*)&k_resolve<M, false>;
+const void* resolve_kernel_t(uint32_t copies) {
+  return copies == 1 ? (const void*)&k_resolve<M, 1> : (const void*)&k_resolve<M, (int)run_copies(M::NS)>;
 }
 template <class M>
 void properties_t(const BatchDev& b, uint32_t run, uint64_t n, uint32_t n_c, double* values, double* spatial,

@@ -54,7 +54,8 @@ def footprint(case, n_var):
     for V, rows, cols, flows in case.maps:
         deg = max(1, int(max(1, (len(flows) + case.n_c - 1) // case.n_c)))
         maps += case.n_c * (8 * 4 + 12 * 2 * deg) + 20 * (len(flows) + case.n_c)
-    liquid = 8 * 6 * case.n_s * case.n_c
+    entries = case.n_s * case.n_c
+    liquid = 8 * (6 + ((8 if case.n_s <= 2 else 2) if entries <= 16384 else 1)) * entries
     return slots * per_slot + maps + liquid
 
 
