@@ -703,23 +703,40 @@ int choose_launch(mcst_engine* e) {
   // window of compartments (particles outside it add to S directly)
   const bool windowed = lds_need > lds_cap;
   const size_t ns_b = sizeof(double) * std::max<uint32_t>(1, (uint32_t)M.ns);
-  // a window is sized so that two blocks fit a CU's LDS (with 1 KB for the
-  // kernel's own shared variables): on the 50 000-compartment lattice two
-  // 512-thread blocks per CU with windows of 2496 compartments took 5.36 ms
-  // per step against 5.59 ms for one block with 3072
+  // a window takes a CU's whole LDS (1 KB left for the kernel's own shared
+  // variables), so that one block of 1024 threads works on each CU: particles
+  // drift out of the window's reach with every move (a step along x of the
+  // 50x50x20 lattice is 1000 compartments), and each of those outside it costs
+  // 4 global atomics.  1.2e7 particles of that lattice: 2.62 ms for 6 steps in
+  // compartment order and 3.52 ms after 700 steps; two blocks of 512 with half
+  // the window 3.24 and 5.33.  Probing runs (256-thread blocks only) keep two
+  // blocks per CU
+  const bool one_block = windowed && !probe;
   size_t win_cap = lds_cap;
   if (windowed && prop.maxSharedMemoryPerMultiProcessor > 2 * 1024)
-    win_cap = std::min(lds_cap, (size_t)prop.maxSharedMemoryPerMultiProcessor / 2 - 1024);
+    win_cap = one_block ? (size_t)prop.maxSharedMemoryPerMultiProcessor - 1024
+                        : std::min(lds_cap, (size_t)prop.maxSharedMemoryPerMultiProcessor / 2 - 1024);
   lds_need = std::min(lds_need, ((windowed ? win_cap : lds_cap) / ns_b) * ns_b);
   bool priv = lds_need > 0;
   if (const char* v = std::getenv("MCST_CONTRIB_LDS")) priv = priv && std::atoi(v) != 0;
   b.acc_w = priv ? (uint32_t)(lds_need / ns_b) : 0u;
   int forced_block = e->tuned_block;
   if (const char* v = std::getenv("MCST_PARTICLE_BLOCK")) forced_block = std::atoi(v);
+  // the block sizes in order of preference among equal numbers of waves: one
+  // block of 512 threads per CU flushes half as often as two of 256 (1e7
+  // particles in 5000 compartments 3140 us for 20 steps against 3198, 250 003
+  // in 1989 of 4 species 1180 against 1308 for 30); a short accumulator costs
+  // little to flush and is spread over more CUs by the smaller block (100 000
+  // particles in 64 compartments 2012 us against 2126 for 100 steps), as is a
+  // batch, whose blocks also flush at each change of run
+  const size_t entries_max = lds_need / sizeof(double);
+  const bool wide = priv && !windowed && live <= 1 && entries_max >= 512;
+  const int order[3] = {wide ? 512 : 256, wide ? 256 : 512, 1024};
   ParticleLaunch best;
   int best_waves = -1;
-  for (int blk : {256, 512, 1024}) {
+  for (int blk : order) {
     if (!priv && blk != 256) continue;
+    if (windowed && probe && blk == 1024) continue;
     if (forced_block && blk != forced_block) continue;
     const void* fn = M.ops->particle_kernel(blk, priv, false, priv && windowed, e->any_leave);
     if (!fn) continue;
@@ -735,13 +752,10 @@ int choose_launch(mcst_engine* e) {
     if (hipFuncGetAttributes(&fa, fn) == hipSuccess && fa.localSizeBytes > 0 && !forced_block)
       per_cu = per_cu / 2;  // register spills: prefer a variant that fits
     // waves per CU count up to 8, and a grid holds at most 8 waves per CU
-    // (but one block of 1024): the pass is bound by the misses a CU's vector
-    // L1 keeps in flight, and more waves only share them (on the
-    // 1e7-particle network 16 waves per CU took 0.204-0.214 ms against 0.167
-    // ms for 8); on a tie the smaller block wins (more blocks, shorter
-    // flushes).  With a compartment window, up to 16 (two 512-thread
-    // blocks): its waves also wait on window flushes and global atomics of
-    // the particles outside the window
+    // (but one block of 1024); with a compartment window up to 16: its waves
+    // also wait on window flushes and the global atomics of the particles
+    // outside it.  Twice the waves: 1e7 particles 3245 us for 20 steps against
+    // 3198, 3e6 particles 2919 against 2922 for 40
     const int wcap = windowed ? 16 : 8;
     const int use = std::min(per_cu, std::max(1, wcap * 64 / blk));
     const int waves = std::min(use * blk / 64, wcap);
@@ -768,11 +782,13 @@ int choose_launch(mcst_engine* e) {
   if (best.probe && best.lds > 64 * 1024)
     (void)hipFuncSetAttribute(M.ops->particle_kernel(256, best.priv, true, best.win, true),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)best.lds);
-  // one run whose accumulator fits: blocks take groups in turn, which keeps
-  // the wave front of the whole grid inside a narrow window of the particle
-  // arrays; a batch, or a window of compartments: one contiguous range per
-  // block, so it meets few runs and few compartments
-  b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : (live <= 1 && !windowed ? 1u : 0u);
+  // one run, or a window of compartments: blocks take groups in turn, which
+  // keeps the wave front of the whole grid inside a narrow window of the
+  // particle arrays (and, with a compartment window, centres it for each
+  // group); a batch takes turns of 4 groups, so that a block changes runs less
+  // often (40 uneven runs of 8.6e6 particles in all, 60 steps: 9164 us, turns
+  // of 2 and 8 10080 and 10180, one contiguous range per block 10090)
+  b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : (live <= 1 || windowed ? 1u : 4u);
   if (const char* v = std::getenv("MCST_TILE_GROUP")) b.tile_group = (uint32_t)std::max(0, std::atoi(v));
   // copies of the accumulators: 8 for a batch of few enough values (each of its
   // runs then has 8 allocated), else one

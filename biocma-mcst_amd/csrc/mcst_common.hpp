@@ -257,7 +257,7 @@ struct BatchDev {
   uint32_t ns_max;          // largest species count of the batch
   uint32_t T_max;
   uint32_t nsub;            // sub-chunks per tile of the model's particle pass, TILE / (64 * M::NL)
-  uint32_t tile_group;      // particle pass: consecutive tiles per block turn (0: one range per block)
+  uint32_t tile_group;      // particle pass: groups per block turn at most (0: one range per block)
   uint32_t acc_w;           // particle pass: compartments per LDS contribution window (PRIV)
   uint32_t stages;
   // copies of each run's contribution accumulator in use (1 or run_copies): block

@@ -314,16 +314,19 @@ __device__ __forceinline__ void add_pair(unsigned long long* w, uint32_t lo, uin
 }
 
 // Adds a block's LDS contribution accumulator, [n_s][win] for compartments
-// [w0, w0 + win) of a run with n_c compartments, to S: one atomic per
-// nonzero entry.
+// [w0, w0 + win) of a run with n_c compartments, to S, and clears it: one
+// atomic per nonzero entry.
 template <int BLK>
-__device__ __forceinline__ void flush_window(const double* s_acc, GLOBAL_AS double* S, uint32_t ns, uint32_t win,
+__device__ __forceinline__ void flush_window(double* s_acc, GLOBAL_AS double* S, uint32_t ns, uint32_t win,
                                              uint32_t n_c, uint32_t w0, uint32_t tid) {
   const uint32_t len = ns * win;
   if (win == n_c) {  // the whole run: the layouts coincide
     for (uint32_t i = tid; i < len; i += BLK) {
       const double v = s_acc[i];
-      if (v != 0.0) unsafeAtomicAdd((double*)(S + i), v);
+      if (v != 0.0) {
+        unsafeAtomicAdd((double*)(S + i), v);
+        s_acc[i] = 0.0;
+      }
     }
     return;
   }
@@ -332,6 +335,7 @@ __device__ __forceinline__ void flush_window(const double* s_acc, GLOBAL_AS doub
     if (v != 0.0) {
       const uint32_t q = i / win;
       unsafeAtomicAdd((double*)(S + (size_t)q * n_c + w0 + (i - q * win)), v);
+      s_acc[i] = 0.0;
     }
   }
 }
@@ -472,8 +476,10 @@ __global__ void __launch_bounds__(BLK)
   const uint32_t T = tile_off[R];
   const uint32_t n_sc = T * NSUB;        // sub-chunks of the pass
   const uint32_t n_groups = (n_sc + WPB - 1) / WPB;
+  // a turn is at most a block's share of the groups, so that every block has
+  // one (8 served runs of 6e5 particles: 12.0 us a pass, 17 with turns of 4)
   const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
-  const uint32_t G = b.tile_group ? b.tile_group : (chunk ? chunk : 1u);
+  const uint32_t G = b.tile_group && b.tile_group < chunk ? b.tile_group : (chunk ? chunk : 1u);
   uint32_t grp = blockIdx.x * G;
   if (grp >= n_groups) return;  // the whole block
   const uint32_t copy = blockIdx.x & (b.n_copies - 1u);  // of each run's accumulator
@@ -628,29 +634,20 @@ __global__ void __launch_bounds__(BLK)
         for (uint32_t i = tid; i < acc_ns * acc_win; i += BLK) s_acc[i] = 0.0;
         __syncthreads();
       } else if constexpr (WIN) {
-        // the window follows the block's slots: when the group's first
-        // compartment leaves the window's lower half (slots are in
-        // compartment order, newborns at the end of the run in parent
-        // order), flush it and re-centre a quarter ahead.  Checked on every
-        // other group (grp is the same in every wave): the check costs two
-        // block barriers, and the window only decides which contributions
-        // take the LDS and which take global atomics.  On the 50 000-
-        // compartment lattice at 1e8 particles, checking every group cost 6 %
-        // of the step; every 8th or 16th let the window lag behind the
-        // newborns and cost more
-        if (acc_win < acc_nc && (grp & 1u) == 0) {
-          if (tid == 0) s_w0 = cur.cnt ? A.pos[0] : acc_w0;
+        // the window follows the block's slots, looked at where a turn of the
+        // block begins (a block barrier per turn): when the turn's first
+        // compartment has left the window's middle half, flush it and centre
+        // it there
+        if (acc_win < acc_nc && grp % G == 0) {
+          if (tid == 0) s_w0 = cur.cnt ? A.pos[0] : acc_w0 + acc_win / 2;
           __syncthreads();
           const uint32_t c0 = s_w0;
           __syncthreads();  // every wave has read s_w0
-          if (c0 - acc_w0 >= acc_win / 2) {  // wraps when below the window
+          if (c0 - (acc_w0 + acc_win / 4) >= acc_win / 2) {  // wraps when below
             flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
-            const uint32_t q = acc_win / 4;
-            const uint32_t lo = c0 > q ? c0 - q : 0u;
+            const uint32_t lo = c0 > acc_win / 2 ? c0 - acc_win / 2 : 0u;
             acc_w0 = lo + acc_win <= acc_nc ? lo : acc_nc - acc_win;
-            __syncthreads();  // the flush has read every entry
-            for (uint32_t i = tid; i < acc_ns * acc_win; i += BLK) s_acc[i] = 0.0;
-            __syncthreads();
+            __syncthreads();  // the flush has cleared every entry
           }
         }
       }
@@ -1563,6 +1560,7 @@ static const void* kernel_ptr_lv(int blk, bool priv, bool win) {
   if (win) {
     if (blk == 256) return (const void*)&k_particle<M, 256, M::NL, lane_interleave(M::NL), true, false, true, LV>;
     if (blk == 512) return (const void*)&k_particle<M, 512, M::NL, lane_interleave(M::NL), true, false, true, LV>;
+    if (blk == 1024) return (const void*)&k_particle<M, 1024, M::NL, lane_interleave(M::NL), true, false, true, LV>;
     return nullptr;
   }
   if (blk == 256) return (const void*)&k_particle<M, 256, M::NL, lane_interleave(M::NL), true, false, false, LV>;
@@ -1589,7 +1587,9 @@ static void launch_lv(const BatchDev& b, const ParticleLaunch& L, hipStream_t s)
   if (!L.priv) {
     launch_particle_t<M, 256, false, false, false, LV>(b, L.grid, 0, s);
   } else if (L.win) {
-    if (L.block == 512)
+    if (L.block == 1024)
+      launch_particle_t<M, 1024, true, false, true, LV>(b, L.grid, L.lds, s);
+    else if (L.block == 512)
       launch_particle_t<M, 512, true, false, true, LV>(b, L.grid, L.lds, s);
     else
       launch_particle_t<M, 256, true, false, true, LV>(b, L.grid, L.lds, s);
