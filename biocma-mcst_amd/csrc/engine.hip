@@ -400,7 +400,8 @@ struct HostRun {
   std::vector<uint32_t> vf;        // time-dependent feeds (indices into feeds), in feed order
   std::vector<uint32_t> vx_out;    // outlets whose first leaving feed is time-dependent ...
   std::vector<uint32_t> vx_feed;   // ... and that feed (index into vf)
-  double* d_vf = nullptr;          // device: this step's flows of vf, then the outlets' thresholds
+  double* d_vf = nullptr;          // device: VF_ROWS rows of a step's flows of vf, then the outlets' thresholds
+  uint32_t vf_from = 0, vf_to = 0; // the steps those rows hold
   double ratio = 0.01;
   uint64_t min_removal = 0;
   uint32_t div_cap = 0xFFFFFFFFu; // newborns per step at most (the reference's division buffer)
@@ -992,8 +993,9 @@ int upload_run(mcst_engine* e, uint32_t r) {
       return run_upload(h, (uint32_t**)dst, v.data(), v.size());
     };
     if (src_c.empty()) src_c.push_back(0.0);
-    std::vector<double> zero_vf(h.vf.size() + h.vx_out.size(), 0.0);
-    if ((rc = run_upload(h, &h.d_vf, zero_vf.data(), zero_vf.size()))) return rc;
+    d.vf_w = (uint32_t)(h.vf.size() + h.vx_out.size());
+    if ((rc = run_alloc(h, (void**)&h.d_vf, (size_t)VF_ROWS * d.vf_w * sizeof(double)))) return rc;
+    h.vf_from = h.vf_to = 0;  // filled before the first step
     d.vf_q = h.d_vf;
     if ((rc = up_u32(&d.vf_src_ptr, sp_ptr))) return rc;
     if ((rc = up_u32(&d.vf_src_k, src_k))) return rc;
@@ -1249,9 +1251,8 @@ void launch_step(mcst_engine* e, uint32_t stages, const hipEvent_t* ev = nullptr
 }
 
 // Whether consecutive steps of a call may run each next step's transport
-// inside the resolve kernel: not when the host writes flows before every
-// step (time-dependent feeds) or may re-lay the runs between steps (growth),
-// and only for whole steps.
+// inside the resolve kernel: not when the host may re-lay the runs between
+// steps (growth), and only for whole steps.
 bool can_transport_ahead(const mcst_engine* e, uint32_t stages);
 
 int read_state(mcst_engine* e, int32_t run, RunState& s) {
@@ -1584,24 +1585,30 @@ void count_steps(mcst_engine* e, uint64_t k) {
 }
 
 // Flows of the time-dependent feeds for the step each live run is about to
-// take (t = step * dt, as update_feed), and the exit thresholds of the
-// outlets they lead, computed on the host like the constant feeds'.
+// take and the one after it, which that step's resolve kernel may transport (t
+// = step * dt, as update_feed), and the exit thresholds of the outlets they
+// lead, computed on the host like the constant feeds': VF_ROWS steps at a time.
 int prepare_feeds(mcst_engine* e) {
   bool synced = false;
   std::vector<double> v;
   for (auto& h : e->runs) {
     if (h.phase != 1 || h.vf.empty() || h.host_step >= h.step_target) continue;
-    if (!synced) {  // the previous step's transport has read the last values
+    if (h.host_step >= h.vf_from && (uint64_t)h.host_step + 2 <= h.vf_to) continue;
+    if (!synced) {  // the steps launched so far have read the rows they need
       HIP_TRY(hipStreamSynchronize(e->stream));
       synced = true;
     }
-    const double t = (double)h.host_step * h.dt;
-    v.assign(h.vf.size() + h.vx_out.size(), 0.0);
-    for (size_t q = 0; q < h.vf.size(); ++q) v[q] = feed_flow(h.feeds[h.vf[q]], t);
-    const HostMap& mp = h.maps[(h.host_step / h.steps_per_map) % h.maps.size()];
-    for (size_t x = 0; x < h.vx_out.size(); ++x) {
-      const uint32_t o = h.vx_out[x];
-      v[h.vf.size() + x] = std::exp(-(h.dt * v[h.vx_feed[x]]) / mp.V[o]);
+    const size_t w = h.vf.size() + h.vx_out.size();
+    v.assign(w * VF_ROWS, 0.0);
+    h.vf_from = h.host_step;
+    h.vf_to = (uint32_t)std::min<uint64_t>((uint64_t)h.host_step + VF_ROWS, 0xFFFFFFFFull);
+    for (uint32_t step = h.vf_from; step < h.vf_to; ++step) {
+      double* row = v.data() + (size_t)(step % VF_ROWS) * w;
+      const double t = (double)step * h.dt;
+      for (size_t q = 0; q < h.vf.size(); ++q) row[q] = feed_flow(h.feeds[h.vf[q]], t);
+      const HostMap& mp = h.maps[(step / h.steps_per_map) % h.maps.size()];
+      for (size_t x = 0; x < h.vx_out.size(); ++x)
+        row[h.vf.size() + x] = std::exp(-(h.dt * row[h.vx_feed[x]]) / mp.V[h.vx_out[x]]);
     }
     HIP_TRY(hipMemcpy(h.d_vf, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice));
   }
@@ -1615,7 +1622,7 @@ bool has_time_feeds(const mcst_engine* e) {
 }
 
 bool can_transport_ahead(const mcst_engine* e, uint32_t stages) {
-  return stages == STAGE_ALL && !has_time_feeds(e) && !has_growth(e);
+  return stages == STAGE_ALL && !has_growth(e);
 }
 
 // One step of the batch, then the reorders that fall due (transported,
@@ -2154,7 +2161,7 @@ int mcst_engine_capture(mcst_engine* e, uint32_t n_steps) {
   if (!e->committed) return fail(MCST_ERR_STATE, "engine not committed");
   if (n_steps == 0) return fail(MCST_ERR_ARG, "capture at least one step");
   if (has_time_feeds(e))
-    return fail(MCST_ERR_STATE, "a run has time-dependent feeds: their flows are set by the host before each step");
+    return fail(MCST_ERR_STATE, "a run has time-dependent feeds: their flows are set by the host ahead of the steps");
   if (has_growth(e)) return fail(MCST_ERR_STATE, "a run grows its capacity: the host checks it between steps");
   HIP_TRY(hipSetDevice(e->device));
   HIP_TRY(hipStreamSynchronize(e->stream));

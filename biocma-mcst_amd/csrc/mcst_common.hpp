@@ -103,6 +103,13 @@ struct MapDev {
 };
 constexpr uint32_t MOVE_ROW_M = 6;
 
+// Steps of time-dependent feeds the host prepares at once: their flows depend
+// on the step number alone.  (Prepared before every step, they cost a wait for
+// the stream and a copy each time, and kept the next step's transport out of
+// the resolve kernel: 20 011 particles of a two-phase column 50 us a step, now
+// 25.)
+constexpr uint32_t VF_ROWS = 256;
+
 // vf_src_s / vf_sink_k entries that belong to the gas phase
 constexpr uint32_t VF_GAS = 0x80000000u;
 
@@ -132,10 +139,11 @@ struct RunDev {
   const double* Fg;         // [n_s][n_c]
   const double* sink_g;     // [n_c]
   double henry[MAX_SPECIES];
-  // time-dependent (linear, exponential) feeds: their flows this step, then
-  // the exit thresholds of the outlets they lead (written by the host before
-  // each step); sources and sinks by compartment (CSR); vx_slot[j] >= 0
-  // selects the threshold of outlet j from vf_q[n_vf + slot]
+  // time-dependent (linear, exponential) feeds: row step % VF_ROWS of vf_q
+  // holds a step's flows, then the exit thresholds of the outlets they lead
+  // (vf_w values, written by the host ahead of the steps); sources and sinks by
+  // compartment (CSR); vx_slot[j] >= 0 selects the threshold of outlet j from
+  // the row's n_vf + slot
   const double* vf_q;
   const uint32_t* vf_src_ptr;  // [n_c+1]
   const uint32_t* vf_src_k;    // feed (index into vf_q) of each source entry
@@ -144,7 +152,7 @@ struct RunDev {
   const uint32_t* vf_sink_ptr; // [n_c+1]
   const uint32_t* vf_sink_k;   // (| VF_GAS for a gas outlet)
   const int32_t* vx_slot;      // [n_c]
-  uint32_t n_vf;
+  uint32_t n_vf, vf_w;
   double* rec;              // [2][n_c][rec_w] per-compartment record read by the particle pass, the
                             // table of step k at k & 1 (the next step's transport may write its
                             // table while this step's resolve kernel reads the other)

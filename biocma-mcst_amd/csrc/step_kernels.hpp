@@ -186,7 +186,8 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
   const MapDev& mp = maps[rd.map_base + (step / rd.steps_per_map) % rd.n_maps];
   const double p_move = gp(mp.p_move)[j];
   double qx = gp(mp.q_exit)[j];
-  if (rd.n_vf && rd.vx_slot[j] >= 0) qx = rd.vf_q[rd.n_vf + (uint32_t)rd.vx_slot[j]];
+  const double* const vf = rd.vf_q + (size_t)(step % VF_ROWS) * rd.vf_w;  // this step's flows (n_vf > 0)
+  if (rd.n_vf && rd.vx_slot[j] >= 0) qx = vf[rd.n_vf + (uint32_t)rd.vx_slot[j]];
   const GLOBAL_AS double* c = gp(rd.C[step & 1u]);
   const bool gas = rd.Cg[0] != nullptr;
   double cn[NS], mn[NS];  // new concentrations and masses
@@ -205,12 +206,12 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
       for (uint32_t q = rd.vf_sink_ptr[j]; q < rd.vf_sink_ptr[j + 1]; ++q) {
         const uint32_t k = rd.vf_sink_k[q];
         if (k & VF_GAS)
-          sink_g = sink_g + rd.vf_q[k & ~VF_GAS];
+          sink_g = sink_g + vf[k & ~VF_GAS];
         else
-          sink = sink + rd.vf_q[k];
+          sink = sink + vf[k];
       }
       for (uint32_t q = rd.vf_src_ptr[j]; q < rd.vf_src_ptr[j + 1]; ++q) {
-        const double add = rd.vf_q[rd.vf_src_k[q]] * rd.vf_src_c[q];
+        const double add = vf[rd.vf_src_k[q]] * rd.vf_src_c[q];
         const uint32_t sp = rd.vf_src_s[q];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {

@@ -150,8 +150,8 @@ int mcst_run_set_steps_per_flowmap(mcst_engine* e, int32_t run, uint32_t steps);
  * adds flow*conc[v] of species[v] at `input`; output >= 0 is a leaving flow.
  * A linear or exponential feed takes t = step*dt at the start of each step
  * (update_feed, simulation.model.cpp:72-122): its flow, and the exit
- * threshold of an outlet it is the first feed of, are set by the host before
- * each step, so an engine holding such a run cannot capture a graph. */
+ * threshold of an outlet it is the first feed of, are set by the host ahead
+ * of the steps, so an engine holding such a run cannot capture a graph. */
 int mcst_run_add_feed(mcst_engine* e, int32_t run, int kind, double f0, double param, uint32_t input,
                       int64_t output, uint32_t n_values, const uint32_t* species, const double* conc);
 /* Initial concentrations [n_species][n_c] (kg/m3); liquid mass = C * V. */
