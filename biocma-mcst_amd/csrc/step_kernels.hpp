@@ -929,156 +929,189 @@ __global__ void __launch_bounds__(BLK)
 // the next pass (n_sc: the sub-chunks of this step's layout).  With `layout`
 // it also lays out the next step's tiles (layout_pass), from the counts it
 // has just computed.
+// What the books read of a run, requested together (before its counter shards
+// are, so that both round trips to memory overlap).
+struct RunBooks {
+  uint32_t n = 0, inactive = 0, step = 0, active = 0;
+  uint32_t cap = 0, div_cap = 0, leave = 0, target = 0;
+  uint64_t min_removal = 0;
+  double ratio = 0.0;
+  unsigned long long cnt[C_COUNT] = {};
+};
+
+__device__ __forceinline__ void read_books(const RunState* rs, const RunDev& rd, RunBooks& k) {
+  k.n = rs->n;
+  k.inactive = rs->inactive;
+  k.step = rs->step;
+  k.active = rs->active;
+#pragma unroll
+  for (int c = 0; c < C_COUNT; ++c) k.cnt[c] = rs->counters[c];
+  k.cap = rd.cap;
+  k.div_cap = rd.div_cap;
+  k.leave = rd.enable_leave;
+  k.target = rd.step_target;
+  k.min_removal = rd.min_removal;
+  k.ratio = rd.ratio;
+}
+
+// The books of one run after its step, from the step's counts (packed as in
+// RunShard).  tiles: of [0, n_end) when the run compacts; tiles_l: of the next
+// step's layout.
+__device__ __forceinline__ void keep_books(const BatchDev& b, RunState* rs, RunBooks& k, unsigned long long mr,
+                                           unsigned long long ed, bool layout, uint32_t& tiles, uint32_t& tiles_l) {
+  uint32_t step_now = k.step, n_now = k.n;  // after this step's books
+  if (k.active) {
+    const uint32_t n = k.n;
+    const unsigned long long moves = (uint32_t)mr, req = mr >> 32;
+    const unsigned long long exits = (uint32_t)ed, deaths = ed >> 32;
+    const unsigned long long processed = n - k.inactive;  // every Idle slot
+    const uint32_t room = k.cap - n;
+    const uint32_t budget = room < k.div_cap ? room : k.div_cap;
+    const uint32_t births = req < budget ? (uint32_t)req : budget;
+    k.cnt[C_BIRTHS] += births;
+    k.cnt[C_EXITS] += exits;
+    k.cnt[C_DEATHS] += deaths;
+    k.cnt[C_MOVES] += moves;
+    k.cnt[C_OVERFLOW] += req - births;
+    k.cnt[C_PROCESSED] += processed;
+    uint64_t inactive = (uint64_t)k.inactive + exits + deaths;
+    const uint64_t thr_ratio = (uint64_t)((double)n * k.ratio);
+    const uint64_t thr = k.min_removal > thr_ratio ? k.min_removal : thr_ratio;
+    const uint32_t n_end = n + births;
+    uint32_t n_keep = n_end, compact = 0;
+    if ((b.stages & STAGE_REMOVE) && inactive > thr) {
+      k.cnt[C_COMPACTIONS] += 1;
+      if (inactive >= n_end) {
+        n_keep = 0;
+        compact = 2;  // everything removed, nothing to move
+      } else {
+        n_keep = n_end - (uint32_t)inactive;
+        compact = 1;
+        tiles = (n_end + TILE - 1u) / TILE;
+      }
+      inactive = 0;
+    }
+    // the age clocks tick with the stages the step ran
+    if (b.stages & STAGE_MODEL) rs->clock_div += 1u;
+    if (k.leave && (b.stages & STAGE_LEAVE)) rs->clock_hyd += 1u;
+    step_now = k.step + 1u;
+    n_now = n_keep;
+    rs->n_end = n_end;
+    rs->n_keep = n_keep;
+    rs->compact = compact;
+    rs->births = births;
+    rs->inactive = (uint32_t)inactive;
+    rs->n = n_keep;
+    rs->step = step_now;
+    k.cnt[C_STEPS] = step_now;
+    k.cnt[C_N] = n_keep;
+    k.cnt[C_INACTIVE] = (uint32_t)inactive;
+#pragma unroll
+    for (int c = 0; c < C_COUNT; ++c) rs->counters[c] = k.cnt[c];
+  } else {
+    rs->compact = 0;
+  }
+  if (layout) {  // layout_pass's table, from the values at hand
+    const uint32_t act = step_now < k.target ? 1u : 0u;
+    tiles_l = act ? (n_now + TILE - 1u) / TILE : 0u;
+    rs->active = act;
+    rs->n_tiles = tiles_l;
+  }
+}
+
 __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs, uint32_t n_sc, bool layout) {
   constexpr uint32_t NT = 256, NWV = NT / 64;
   __shared__ uint32_t s_w[NWV], s_wl[NWV];
   __shared__ uint32_t s_carry, s_carry_l;
   __shared__ unsigned long long s_mr[NT], s_ed[NT];  // the counts of 256 runs, summed over their shards
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  if (tid == 0) s_carry = s_carry_l = 0;
   const uint32_t nsh = b.n_shard;
-  for (uint32_t r0 = 0; r0 < b.R; r0 += NT) {
-    const uint32_t r = r0 + tid;
-    // what the books read of the run's state, requested before the shards so
-    // that both round trips to memory overlap
-    RunState* const rs = b.rs + r;
-    uint32_t n = 0, inactive0 = 0, step0 = 0, active = 0;
-    uint32_t cap = 0, div_cap = 0, leave = 0, target = 0;
-    uint64_t min_removal = 0;
-    double ratio = 0.0;
-    unsigned long long cnt[C_COUNT] = {};
-    if (r < b.R) {
-      const RunDev& rd = runs[r];
-      n = rs->n;
-      inactive0 = rs->inactive;
-      step0 = rs->step;
-      active = rs->active;
-#pragma unroll
-      for (int k = 0; k < C_COUNT; ++k) cnt[k] = rs->counters[k];
-      cap = rd.cap;
-      div_cap = rd.div_cap;
-      leave = rd.enable_leave;
-      target = rd.step_target;
-      min_removal = rd.min_removal;
-      ratio = rd.ratio;
+  // read and reset with atomics: other blocks added to the shards with
+  // atomics up to a moment ago.  One lane per shard, all in flight at once;
+  // both halves of a sum stay below 2^32 (a run has fewer slots)
+  auto take = [&](uint32_t i, uint32_t n, unsigned long long& mr, unsigned long long& ed) {
+    mr = ed = 0;
+    if (i < n) {
+      mr = atomicExch(&b.shards[i].moves_requests, 0ull);
+      ed = atomicExch(&b.shards[i].exits_deaths, 0ull);
     }
-    // read and reset with atomics: other blocks added to the shards with
-    // atomics up to a moment ago.  One lane per shard, all in flight at once
-    const uint32_t n_run = b.R - r0 < NT ? b.R - r0 : NT;
-    for (uint32_t i0 = 0; i0 < n_run * nsh; i0 += NT) {
-      const uint32_t i = i0 + tid;
-      unsigned long long mr = 0, ed = 0;
-      if (i < n_run * nsh) {
-        RunShard* sh = b.shards + (size_t)r0 * nsh + i;
-        mr = atomicExch(&sh->moves_requests, 0ull);
-        ed = atomicExch(&sh->exits_deaths, 0ull);
-      }
-      // both halves stay below 2^32 (a run has fewer slots): no carry between them
-      for (uint32_t d = nsh >> 1; d; d >>= 1) {
-        mr += __shfl_xor(mr, (int)d, 64);
-        ed += __shfl_xor(ed, (int)d, 64);
-      }
-      if (i < n_run * nsh && i % nsh == 0) {
-        s_mr[i / nsh] = mr;
-        s_ed[i / nsh] = ed;
-      }
+    for (uint32_t d = nsh >> 1; d; d >>= 1) {
+      mr += __shfl_xor(mr, (int)d, 64);
+      ed += __shfl_xor(ed, (int)d, 64);
     }
-    __syncthreads();
-    uint32_t tiles = 0;   // tiles of [0, n_end) when the run compacts
-    uint32_t tiles_l = 0; // tiles of the next step's layout
-    if (r < b.R) {
-      uint32_t step_now = step0, n_now = n;  // after this step's books
-      if (active) {
-        const unsigned long long moves = (uint32_t)s_mr[tid], req = s_mr[tid] >> 32;
-        const unsigned long long exits = (uint32_t)s_ed[tid], deaths = s_ed[tid] >> 32;
-        const unsigned long long processed = n - inactive0;  // every Idle slot
-        const uint32_t room = cap - n;
-        const uint32_t budget = room < div_cap ? room : div_cap;
-        const uint32_t births = req < budget ? (uint32_t)req : budget;
-        cnt[C_BIRTHS] += births;
-        cnt[C_EXITS] += exits;
-        cnt[C_DEATHS] += deaths;
-        cnt[C_MOVES] += moves;
-        cnt[C_OVERFLOW] += req - births;
-        cnt[C_PROCESSED] += processed;
-        uint64_t inactive = (uint64_t)inactive0 + exits + deaths;
-        const uint64_t thr_ratio = (uint64_t)((double)n * ratio);
-        const uint64_t thr = min_removal > thr_ratio ? min_removal : thr_ratio;
-        const uint32_t n_end = n + births;
-        uint32_t n_keep = n_end, compact = 0;
-        if ((b.stages & STAGE_REMOVE) && inactive > thr) {
-          cnt[C_COMPACTIONS] += 1;
-          if (inactive >= n_end) {
-            n_keep = 0;
-            compact = 2;  // everything removed, nothing to move
-          } else {
-            n_keep = n_end - (uint32_t)inactive;
-            compact = 1;
-            tiles = (n_end + TILE - 1u) / TILE;
-          }
-          inactive = 0;
+  };
+  if (b.R == 1) {  // one run: no scan over runs, no barrier (1 us of a step)
+    if (wave == 0) {
+      RunBooks k;
+      if (lane == 0) read_books(b.rs, runs[0], k);
+      unsigned long long mr, ed;
+      take(lane, nsh, mr, ed);
+      if (lane == 0) {
+        uint32_t tiles = 0, tiles_l = 0;
+        keep_books(b, b.rs, k, mr, ed, layout, tiles, tiles_l);
+        b.rm_tile_off[0] = 0u;
+        b.rm_tile_off[1] = tiles;
+        if (layout) {
+          b.tile_off[0] = 0u;
+          b.tile_off[1] = tiles_l;
+          b.rs[0].tile_begin = 0u;
         }
-        // the age clocks tick with the stages the step ran
-        if (b.stages & STAGE_MODEL) rs->clock_div += 1u;
-        if (leave && (b.stages & STAGE_LEAVE)) rs->clock_hyd += 1u;
-        step_now = step0 + 1u;
-        n_now = n_keep;
-        rs->n_end = n_end;
-        rs->n_keep = n_keep;
-        rs->compact = compact;
-        rs->births = births;
-        rs->inactive = (uint32_t)inactive;
-        rs->n = n_keep;
-        rs->step = step_now;
-        cnt[C_STEPS] = step_now;
-        cnt[C_N] = n_keep;
-        cnt[C_INACTIVE] = (uint32_t)inactive;
-#pragma unroll
-        for (int k = 0; k < C_COUNT; ++k) rs->counters[k] = cnt[k];
-      } else {
-        rs->compact = 0;
-      }
-      if (layout) {  // layout_pass's table, from the values at hand
-        const uint32_t act = step_now < target ? 1u : 0u;
-        tiles_l = act ? (n_now + TILE - 1u) / TILE : 0u;
-        rs->active = act;
-        rs->n_tiles = tiles_l;
       }
     }
-    const uint32_t inc = wave_incl_scan(tiles, lane);
-    const uint32_t inc_l = layout ? wave_incl_scan(tiles_l, lane) : 0u;
-    if (lane == 63) {
-      s_w[wave] = inc;
-      s_wl[wave] = inc_l;
-    }
-    __syncthreads();
-    uint32_t wpre = 0, tot = 0, wpre_l = 0, tot_l = 0;
-    for (uint32_t w = 0; w < NWV; ++w) {
-      if (w < wave) {
-        wpre += s_w[w];
-        wpre_l += s_wl[w];
+  } else {
+    if (tid == 0) s_carry = s_carry_l = 0;
+    for (uint32_t r0 = 0; r0 < b.R; r0 += NT) {
+      const uint32_t r = r0 + tid;
+      RunBooks k;
+      if (r < b.R) read_books(b.rs + r, runs[r], k);
+      const uint32_t n_run = b.R - r0 < NT ? b.R - r0 : NT;
+      for (uint32_t i0 = 0; i0 < n_run * nsh; i0 += NT) {
+        const uint32_t i = i0 + tid;
+        unsigned long long mr, ed;
+        take(r0 * nsh + i, (r0 + n_run) * nsh, mr, ed);
+        if (i < n_run * nsh && i % nsh == 0) {
+          s_mr[i / nsh] = mr;
+          s_ed[i / nsh] = ed;
+        }
       }
-      tot += s_w[w];
-      tot_l += s_wl[w];
-    }
-    const uint32_t carry = s_carry, carry_l = s_carry_l;
-    if (r < b.R) {
-      b.rm_tile_off[r] = carry + wpre + inc - tiles;
-      if (layout) {
-        b.tile_off[r] = carry_l + wpre_l + inc_l - tiles_l;
-        b.rs[r].tile_begin = carry_l + wpre_l + inc_l - tiles_l;
+      __syncthreads();
+      uint32_t tiles = 0, tiles_l = 0;
+      if (r < b.R) keep_books(b, b.rs + r, k, s_mr[tid], s_ed[tid], layout, tiles, tiles_l);
+      const uint32_t inc = wave_incl_scan(tiles, lane);
+      const uint32_t inc_l = layout ? wave_incl_scan(tiles_l, lane) : 0u;
+      if (lane == 63) {
+        s_w[wave] = inc;
+        s_wl[wave] = inc_l;
       }
+      __syncthreads();
+      uint32_t wpre = 0, tot = 0, wpre_l = 0, tot_l = 0;
+      for (uint32_t w = 0; w < NWV; ++w) {
+        if (w < wave) {
+          wpre += s_w[w];
+          wpre_l += s_wl[w];
+        }
+        tot += s_w[w];
+        tot_l += s_wl[w];
+      }
+      const uint32_t carry = s_carry, carry_l = s_carry_l;
+      if (r < b.R) {
+        b.rm_tile_off[r] = carry + wpre + inc - tiles;
+        if (layout) {
+          b.tile_off[r] = carry_l + wpre_l + inc_l - tiles_l;
+          b.rs[r].tile_begin = carry_l + wpre_l + inc_l - tiles_l;
+        }
+      }
+      __syncthreads();
+      if (tid == 0) {
+        s_carry = carry + tot;
+        s_carry_l = carry_l + tot_l;
+      }
+      __syncthreads();
     }
-    __syncthreads();
     if (tid == 0) {
-      s_carry = carry + tot;
-      s_carry_l = carry_l + tot_l;
+      b.rm_tile_off[b.R] = s_carry;
+      if (layout) b.tile_off[b.R] = s_carry_l;
     }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    b.rm_tile_off[b.R] = s_carry;
-    if (layout) b.tile_off[b.R] = s_carry_l;
   }
   for (uint32_t i = tid; i < (n_sc + 63u) >> 6; i += NT) b.div_l1[i] = 0u;
   for (uint32_t i = tid; i < (n_sc + 4095u) >> 12; i += NT) b.div_l2[i] = 0u;
