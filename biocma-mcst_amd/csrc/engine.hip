@@ -732,14 +732,22 @@ int choose_launch(mcst_engine* e) {
   // batch, whose blocks also flush at each change of run
   const size_t entries_max = lds_need / sizeof(double);
   const bool wide = priv && !windowed && live <= 1 && entries_max >= 512;
-  const int order[3] = {wide ? 512 : 256, wide ? 256 : 512, 1024};
+  // a small pool of slots: the pass with one slot per lane, which moves its
+  // movers itself
+  const bool small = priv && !windowed && !probe && b.T_max <= small_tiles(M.nv, M.nl);
+  // (its blocks take few turns, so those that flush a long accumulator are the
+  // largest: 345 679 particles in 777 compartments 1177 us for 50 steps against
+  // 1310 with 512 threads and 1557 with 256)
+  const int order[3] = {wide ? (small ? 1024 : 512) : 256, wide ? (small ? 512 : 256) : 512, wide && small ? 256 : 1024};
+  b.moved = small ? 1u : 0u;
+  b.nsub = TILE / (64u * (small ? 1u : (uint32_t)M.nl));
   ParticleLaunch best;
   int best_waves = -1;
   for (int blk : order) {
     if (!priv && blk != 256) continue;
     if (windowed && probe && blk == 1024) continue;
     if (forced_block && blk != forced_block) continue;
-    const void* fn = M.ops->particle_kernel(blk, priv, false, priv && windowed, e->any_leave);
+    const void* fn = M.ops->particle_kernel(blk, priv, false, priv && windowed, e->any_leave, small);
     if (!fn) continue;
     const size_t lds = priv ? lds_need : 0;
     if (lds > 64 * 1024)
@@ -757,7 +765,7 @@ int choose_launch(mcst_engine* e) {
     // also wait on window flushes and the global atomics of the particles
     // outside it.  Twice the waves: 1e7 particles 3245 us for 20 steps against
     // 3198, 3e6 particles 2919 against 2922 for 40
-    const int wcap = windowed ? 16 : 8;
+    const int wcap = windowed || small ? 16 : 8;
     const int use = std::min(per_cu, std::max(1, wcap * 64 / blk));
     const int waves = std::min(use * blk / 64, wcap);
     if (per_cu > 0 && waves > best_waves) {
@@ -772,16 +780,19 @@ int choose_launch(mcst_engine* e) {
   if (best_waves < 0) {  // no resident configuration with the accumulator: go direct
     best = ParticleLaunch{};
     b.acc_w = 0;
+    b.moved = 0;
+    b.nsub = TILE / (64u * (uint32_t)M.nl);
     int per_cu = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, M.ops->particle_kernel(256, false, false, false, e->any_leave), 256, 0));
+        &per_cu, M.ops->particle_kernel(256, false, false, false, e->any_leave, false), 256, 0));
     best.grid = std::min(std::max(per_cu, 1), 2) * prop.multiProcessorCount;  // 8 waves per CU
   }
-  best.grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)best.grid, b.T_max));
+  const uint64_t groups = b.moved ? (uint64_t)b.T_max * b.nsub * 64 / best.block : b.T_max;  // at most
+  best.grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)best.grid, groups));
   best.probe = probe;
   best.leave = e->any_leave;
   if (best.probe && best.lds > 64 * 1024)
-    (void)hipFuncSetAttribute(M.ops->particle_kernel(256, best.priv, true, best.win, true),
+    (void)hipFuncSetAttribute(M.ops->particle_kernel(256, best.priv, true, best.win, true, false),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)best.lds);
   // one run, or a window of compartments: blocks take groups in turn, which
   // keeps the wave front of the whole grid inside a narrow window of the
@@ -1122,6 +1133,11 @@ RequestLevels request_levels(uint64_t T, uint32_t nsub) {
   return RequestLevels{(n_sc + 63) >> 6, (n_sc + 4095) >> 12, (n_sc >> 18) + 1};
 }
 
+// Sub-chunks per tile that a pool of T tiles has list segments for.
+uint32_t list_subs(const ModelEntry& m, uint64_t T) {
+  return T <= small_tiles(m.nv, m.nl) ? NSUB_MAX : TILE / (64u * (uint32_t)m.nl);
+}
+
 int commit(mcst_engine* e) {
   const ModelEntry& M = *e->model;
   const uint32_t R0 = (uint32_t)e->runs.size();
@@ -1140,7 +1156,9 @@ int commit(mcst_engine* e) {
   b.T_max = (uint32_t)T_max;
   b.R = 0;
   b.n_comp_total = 0;
-  b.nsub = TILE / (64u * (uint32_t)M.nl);
+  // lists sized for the particle pass with the most sub-chunks per tile that
+  // the pool may use (choose_launch)
+  b.nsub = list_subs(M, T_max);
   b.ns_max = std::max<uint32_t>(1, (uint32_t)M.ns);  // one model per engine; thread s == 0 also writes the map fields
   b.stages = STAGE_ALL;
   e->runs_cap = std::max(R0, e->reserve_runs);
@@ -1425,7 +1443,8 @@ int grow_pool(mcst_engine* e, uint64_t min_tiles) {
   const uint64_t T1 = std::max<uint64_t>(min_tiles, 2 * T0), P1 = T1 * TILE;
   if (P1 >= 0xFFFFFFFFull) return fail(MCST_ERR_MEMORY, "more than 2^32-1 particle slots in one engine");
   const uint64_t nv = (uint64_t)e->model->nv;
-  const RequestLevels lv = request_levels(T1, b.nsub);
+  const uint32_t nsub = list_subs(*e->model, T1);
+  const RequestLevels lv = request_levels(T1, nsub);
   struct Move {
     void** slot;     // the BatchDev field
     size_t bytes;    // new size
@@ -1449,9 +1468,9 @@ int grow_pool(mcst_engine* e, uint64_t min_tiles) {
       {(void**)&b.move_rec, P1 * 4, 0, 0, nullptr},
       {(void**)&b.div_rec, P1 * 4, 0, 0, nullptr},
       {(void**)&b.div_pos, P1 * 4, 0, 0, nullptr},
-      {(void**)&b.div_stage, T1 * b.nsub * DIV_STAGE * nv * 8, 0, 0, nullptr},
-      {(void**)&b.sub_moves, T1 * b.nsub * 4, 0, 0, nullptr},
-      {(void**)&b.sub_divs, T1 * b.nsub * 4, 0, 0, nullptr},
+      {(void**)&b.div_stage, T1 * nsub * DIV_STAGE * nv * 8, 0, 0, nullptr},
+      {(void**)&b.sub_moves, T1 * nsub * 4, 0, 0, nullptr},
+      {(void**)&b.sub_divs, T1 * nsub * 4, 0, 0, nullptr},
   };
   for (auto& m : mv) {
     const hipError_t err = hipMalloc(&m.fresh, m.bytes);

@@ -33,7 +33,7 @@ struct ParticleLaunch {
 struct ModelOps {
   void (*transport)(const BatchDev& b, int grid, hipStream_t s);
   void (*particle)(const BatchDev& b, const ParticleLaunch& L, hipStream_t s);
-  const void* (*particle_kernel)(int block, bool priv, bool probe, bool win, bool leave);
+  const void* (*particle_kernel)(int block, bool priv, bool probe, bool win, bool leave, bool small);
   // resolve: grid blocks plus aux blocks first in the grid, which take the
   // pass's contributions, for the next step's transport (ahead) or into S
   void (*resolve)(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s);

@@ -22,9 +22,10 @@ constexpr uint32_t TILE = BLOCK * PPT;     // 1024 slots per tile (the reference
 // 3 % faster at 4 slots per lane (pair-wise 16-byte accesses, half the load
 // instructions, were slower), consecutive 4 % faster at 2.
 constexpr bool lane_interleave(int nl) { return nl >= 4; }
-constexpr uint32_t NSUB_MAX = TILE / 128;  // sub-chunks (the pass's unit of work) per tile: TILE / (64 * M::NL)
+constexpr uint32_t NSUB_MAX = TILE / 64;   // sub-chunks (the pass's unit of work) per tile: TILE / (64 * M::NL), 16 in
+                                           // a small batch's pass
 constexpr uint32_t WAVES = BLOCK / 64;
-constexpr uint32_t RESOLVE_GROUP_MAX = 64;  // sub-chunks per group of the resolve kernel: 32 or 64 (at most 256)
+constexpr uint32_t RESOLVE_GROUP_MAX = 128; // sub-chunks per group of the resolve kernel: 32 or 64, 128 of 64 slots
 constexpr uint32_t RESOLVE_TICKETS = 64;    // sub-counters of the resolve kernel's done-count
 constexpr uint32_t TICKET_STRIDE = 32;      // words between two of those counters (a line each)
 constexpr uint32_t REMOVE_RUN_TILES = 512;  // largest capacity at which one block removes a run's inactive slots
@@ -46,6 +47,15 @@ constexpr uint32_t MOVER_INACTIVE = 1u << 10;
 constexpr uint32_t LIST_POS_SHIFT = 11;
 constexpr uint32_t LIST_POS_FAR = 0xFFFFFFFFu >> LIST_POS_SHIFT;
 static_assert(TILE <= MOVER_INACTIVE, "a tile-local slot fits below the flag");
+
+// Largest pool, in tiles, that the small batch's particle pass serves.  Measured
+// per step against the pipelined pass: 100 000 particles of 2 states 15.0 us
+// against 19.6, 345 679 of 3 23.5 and 25.4, 250 003 of 8 (2 slots per lane) 40.2
+// and 40.5, and level at 1e6 (27-50 us).  Where the pipelined pass holds many
+// states of 4 slots per lane its registers leave it few waves and the line lies
+// further up: 1e6 of 6 states 37.3 and 41.8 us, 1e6 of 9 58.5 and 72.9, 3e6 of 9
+// 181 and 157.
+constexpr uint32_t small_tiles(int nv, int nl) { return nv * nl >= 24 ? 3072u : 1024u; }
 
 // Stage mask of one step (values shared with the C ABI).
 enum Stage : uint32_t {
@@ -264,7 +274,8 @@ struct BatchDev {
   uint32_t n_comp_total;
   uint32_t ns_max;          // largest species count of the batch
   uint32_t T_max;
-  uint32_t nsub;            // sub-chunks per tile of the model's particle pass, TILE / (64 * M::NL)
+  uint32_t nsub;            // sub-chunks per tile of the particle pass in use
+  uint32_t moved;           // the small batch's pass is in use: it moves its movers itself
   uint32_t tile_group;      // particle pass: groups per block turn at most (0: one range per block)
   uint32_t acc_w;           // particle pass: compartments per LDS contribution window (PRIV)
   uint32_t stages;

@@ -364,6 +364,10 @@ __device__ __forceinline__ uint32_t cdf_column(const GLOBAL_AS double* cp, uint3
   return left;
 }
 
+// Where a particle that leaves compartment `pos` goes: the first column of its
+// cumulative row at or above u (move_kernel.hpp:61-103).
+__device__ __forceinline__ uint32_t next_place(const MapDev& mp, uint32_t pos, double u);
+
 // Loads and stores of the NL consecutive slots of one lane: 8-byte fields
 // move in 16-byte accesses per lane when NL > 1 (aligned: every run's slots
 // start on a tile boundary), 4-byte fields in one access of 4*NL bytes.
@@ -429,6 +433,22 @@ __device__ __forceinline__ void st_status(GLOBAL_AS uint8_t* p, uint32_t v) {
     *(GLOBAL_AS uint16_t*)p = (uint16_t)v;
   else
     *(GLOBAL_AS uint32_t*)p = v;
+}
+
+__device__ __forceinline__ uint32_t next_place(const MapDev& mp, uint32_t pos, double u) {
+  if (mp.move_row) {  // the compartment's 64-byte record: 5 cdf columns, 6 neighbours
+    const GLOBAL_AS u32x4* rw = (const GLOBAL_AS u32x4*)(gp(mp.move_row) + (size_t)pos * 16);
+    const u32x4 q0 = rw[0], q1 = rw[1], q2 = rw[2], q3 = rw[3];
+    const uint32_t col = (u > __hiloint2double((int)q0.y, (int)q0.x) ? 1u : 0u) +
+                         (u > __hiloint2double((int)q0.w, (int)q0.z) ? 1u : 0u) +
+                         (u > __hiloint2double((int)q1.y, (int)q1.x) ? 1u : 0u) +
+                         (u > __hiloint2double((int)q1.w, (int)q1.z) ? 1u : 0u) +
+                         (u > __hiloint2double((int)q2.y, (int)q2.x) ? 1u : 0u);
+    return col == 0 ? q2.z : col == 1 ? q2.w : col == 2 ? q3.x : col == 3 ? q3.y : col == 4 ? q3.z : q3.w;
+  }
+  const uint32_t m = mp.m;
+  const uint32_t col = cdf_column(gp(mp.cdf) + (size_t)pos * m, m, u);
+  return gp(mp.nbr)[(size_t)pos * m + col];
 }
 
 // The particle pass.  The unit of work is a sub-chunk of SUB = 64*NL slots;
@@ -921,6 +941,169 @@ __global__ void __launch_bounds__(BLK)
   for (int lvl = 0; lvl < 3; ++lvl) flush_requests(lvl);
 }
 
+// The particle pass of a small batch (b.moved; small_tiles).  Such a pass is
+// not bound by memory but by the length of one wave's work from the launch to
+// its last store, so it is cut shorter, not wider: one
+// slot per lane (a sub-chunk is 64 slots; with 4 the model and the draws of a
+// wave took 2 us and the contributions of a wave up to 2.5), no pipeline across
+// sub-chunks (a wave mostly has one), and a mover is moved here instead of in
+// k_resolve, whose group scan, list and chain of loads took 3.8 us more: its
+// row is requested before the model's arithmetic.  Plain loads and stores: the
+// state stays in cache from step to step.  Pass and resolve of 100 000 particles
+// of 2 states in 64 compartments 8.7 and 7.9 us before, 5.6 and 6.6 now.
+template <class M, int BLK, bool LV>
+__global__ void __launch_bounds__(BLK)
+    k_particle_small(BatchDev b, const RunDev* __restrict__ runs, const RunState* __restrict__ rsr,
+                     const MapDev* __restrict__ maps, const uint32_t* __restrict__ tile_off) {
+  constexpr int NV = M::NV, NS = M::NS, NR = record_terms<M>(), REC = rec_stride(NR);
+  constexpr int NQ = NR + 2, NG = LV ? NQ : NQ - 1;
+  constexpr int NP = M::NP > 0 ? M::NP : 1;
+  constexpr uint32_t WPB = BLK / 64, SUB = 64, NSUB = TILE / SUB;
+  extern __shared__ double s_acc[];  // [n_s][n_c] of run acc_run
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uniform(tid >> 6);
+  const uint32_t stages = b.stages, R = b.R;
+  const uint64_t P = b.P;
+  const uint32_t n_sc = tile_off[R] * NSUB;
+  const uint32_t n_groups = (n_sc + WPB - 1) / WPB;
+  // groups dealt to the blocks one at a time; in a batch one range per block,
+  // which meets few runs
+  const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
+  const uint32_t g_first = R == 1 ? blockIdx.x : blockIdx.x * chunk, g_step = R == 1 ? gridDim.x : 1u;
+  const uint32_t g_end = R == 1 || n_groups - g_first < chunk ? n_groups : g_first + chunk;
+  if (g_first >= n_groups) return;
+  const uint32_t copy = blockIdx.x & (b.n_copies - 1u);
+  const bool do_model = (stages & STAGE_MODEL) != 0;
+  const bool do_contrib = (stages & STAGE_CONTRIB) != 0;
+  uint32_t acc_run = 0xFFFFFFFFu, acc_ns = 0, acc_nc = 0;
+  GLOBAL_AS double* acc_S = nullptr;
+  for (uint32_t grp = g_first; grp < g_end; grp += g_step) {
+    // ---- the wave's sub-chunk; none past the last (every wave meets the
+    // block's barriers)
+    const uint32_t sc = grp * WPB + wave;
+    const bool on = sc < n_sc;
+    const uint32_t t = on ? sc / NSUB : 0u;
+    const uint32_t r = on ? find_run(tile_off, R, t) : 0u;
+    const RunDev& rd = runs[r];
+    const uint32_t slot0 = on ? (t - tile_off[r]) * TILE + (sc % NSUB) * SUB : 0u;
+    const uint32_t n = on ? rsr[r].n : 0u;
+    const bool valid = slot0 + lane < n;  // its lane's slot holds a particle
+    const uint32_t slot = valid ? slot0 + lane : 0u;
+    const uint64_t g = rd.p_off + slot;
+    uint32_t st = EXIT, pos = 0;
+    double x[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) x[v] = 0.0;
+    if (valid) {
+      st = gp(b.status)[g];
+      pos = gp(b.pos)[g];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) x[v] = gp(b.state)[(uint64_t)v * P + g];
+    }
+    // ---- block-uniform: the run whose contributions the LDS accumulates
+    const uint32_t r0 = find_run(tile_off, R, (grp * WPB) / NSUB);
+    if (r0 != acc_run) {
+      __syncthreads();
+      flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
+      acc_run = r0;
+      acc_ns = runs[r0].n_s;
+      acc_nc = runs[r0].n_c;
+      acc_S = gp(runs[r0].Sp) + (size_t)copy * acc_ns * acc_nc;
+      for (uint32_t i = tid; i < acc_ns * acc_nc; i += BLK) s_acc[i] = 0.0;
+      __syncthreads();
+    }
+    if (!on) continue;
+    const uint32_t step = rsr[r].step;
+    const uint32_t n_c = rd.n_c;
+    const double dt = rd.dt, w = rd.weight;
+    const bool do_move = rd.enable_move && (stages & STAGE_MOVE);
+    const bool do_leave = LV && rd.enable_leave && (stages & STAGE_LEAVE);
+    const uint32_t clk_d = rsr[r].clock_div + (do_model ? 1u : 0u);
+    const uint32_t clk_h0 = rsr[r].clock_hyd;
+    const MapDev& mp = maps[rd.map_base + (step / rd.steps_per_map) % rd.n_maps];
+    const GLOBAL_AS double* const rec = gp(rd.rec) + ((step & 1u) ? (size_t)n_c * REC : (size_t)0);
+    double rr[NQ];
+#pragma unroll
+    for (int f = 0; f < NG; ++f) rr[f] = valid ? rec[(size_t)pos * REC + f] : 0.0;
+    if constexpr (!LV) rr[NQ - 1] = 1.0;
+    double p[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) p[q] = rd.params[q];
+
+    // ---- the particle: draws, move, model
+    const U4 u = draw4(rd.seed, slot, step, TAG_TRANSPORT, 0u);
+    const bool idle = valid && st == IDLE;
+    const bool mover = valid && do_move && rr[NR] > u01(u.x);  // whatever its status
+    uint32_t to = pos;
+    if (mover) to = next_place(mp, pos, u01(u.y));
+    bool want = false, dead = false, exited = false;
+    double contrib[NS];
+#pragma unroll
+    for (int q = 0; q < NS; ++q) contrib[q] = 0.0;
+    if (idle && do_model) {
+      const int code = M::update(p, dt, x, rr, contrib);
+      if constexpr (M::CAN_DIE) dead = code == DEAD;
+      want = code == DIVISION;
+    }
+    if (do_contrib && idle && !dead) {
+#pragma unroll
+      for (int q = 0; q < NS; ++q) {
+        const double c = w * contrib[q];
+        if (r == acc_run)
+          atomicAdd(s_acc + q * n_c + pos, c);
+        else
+          unsafeAtomicAdd((double*)(gp(rd.Sp) + ((size_t)copy * NS + q) * n_c + pos), c);
+      }
+    }
+    if (do_leave && idle && !dead) {  // the exit test in the compartment it is in now
+      const double qx = mover ? rec[(size_t)to * REC + NR + 1] : rr[NR + 1];
+      exited = qx < 1.0 && u01(u.z) > qx;
+    }
+    // ---- division requests of the sub-chunk, as in k_particle
+    const uint64_t wd = __ballot(want), mv = __ballot(mover);
+    const uint32_t n_div = (uint32_t)__popcll(wd);
+    const uint32_t rk = (uint32_t)__popcll(wd & lanemask_lt(lane));
+    if (n_div) {
+      const uint64_t seg = (uint64_t)sc * SUB;
+      if (want) {
+        if (rk < DIV_STAGE) {
+          GLOBAL_AS double* stg = gp(b.div_stage) + ((uint64_t)sc * DIV_STAGE + rk) * NV;
+#pragma unroll
+          for (int v = 0; v < NV; ++v) stg[v] = x[v];
+          double xd[NV];
+          M::division(p, x, xd, RngKey{rd.seed, slot, step});
+        }
+        const uint32_t pv = pos < LIST_POS_FAR ? pos : LIST_POS_FAR;
+        gp(b.div_rec)[seg + rk] = (slot % TILE) | (pv << LIST_POS_SHIFT);
+        gp(b.div_pos)[seg + rk] = pos;
+      }
+      // (a small pool's one entry of 2^18 sub-chunks is never read)
+      if (lane < 2) atomicAdd((lane ? b.div_l2 : b.div_l1) + (sc >> (lane ? 12 : 6)), n_div);
+    }
+    // ---- stores
+    if (valid) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) gp(b.state)[(uint64_t)v * P + g] = x[v];
+    }
+    if (mover) gp(b.pos)[g] = to;
+    if (exited || dead) {
+      gp(b.status)[g] = dead ? (uint8_t)DEAD : (uint8_t)EXIT;
+      GLOBAL_AS double* a_h = gp(b.age_hyd) + g;
+      GLOBAL_AS uint32_t* c_h = gp(b.clk_hyd) + g;
+      *a_h = dead ? clock_age(*a_h, clk_h0, *c_h, dt) : 0.0;
+      *c_h = clk_d;
+    }
+    const uint32_t n_exit = LV ? (uint32_t)__popcll(__ballot(exited)) : 0u;
+    const uint32_t n_dead = M::CAN_DIE ? (uint32_t)__popcll(__ballot(dead)) : 0u;
+    if (lane == 0) {
+      gp(b.sub_moves)[sc] = (uint32_t)__popcll(mv);
+      gp(b.sub_divs)[sc] = n_div;
+      add_pair(&run_shard(b, r)->exits_deaths, n_exit, n_dead);
+    }
+  }
+  __syncthreads();
+  flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
+}
+
 // The books of every run after its step, kept by the last block of
 // k_resolve: counters, births (the accepted requests), the removal decision
 // of update_and_remove_inactive (particles_container.hpp:539-557, threshold
@@ -1196,8 +1379,9 @@ __global__ void __launch_bounds__(256, M::NV <= 8 ? 4 : 1) k_resolve(BatchDev b,
   const uint32_t n_res = gridDim.x - tr_blocks;  // blocks of the resolve work
   const bool tr_block = blockIdx.x < tr_blocks;
   const uint32_t rb = tr_block ? 0u : blockIdx.x - tr_blocks;  // index among the resolve blocks
-  uint32_t GS = 32;
-  while (GS < RES_SC && (n_sc + 2 * GS - 1) / (2 * GS) >= n_res) GS *= 2;
+  // A small batch's groups hold 128 sub-chunks of 64 slots, whose movers are done.
+  uint32_t GS = nsub > 8 ? RES_SC : 32;
+  while (GS < 64 && (n_sc + 2 * GS - 1) / (2 * GS) >= n_res) GS *= 2;
   const uint32_t n_groups = (n_sc + GS - 1) / GS;
   uint32_t ev_run = 0, ev_moves = 0, ev_req = 0;  // movers and requests of the block's groups (thread 0)
   const bool leave_stage = (b.stages & STAGE_LEAVE) != 0;
@@ -1239,6 +1423,7 @@ __global__ void __launch_bounds__(256, M::NV <= 8 ? 4 : 1) k_resolve(BatchDev b,
     __syncthreads();
     // ---- movers
     const uint32_t total = s_pre[GS];
+    const uint32_t to_move = b.moved ? 0u : total;
     // the step's moves and requests, from the lists: one atomic per block and
     // run, or per sub-chunk where the group holds several runs
     const uint32_t g_last = n_sc - sc0 < GS ? n_sc - sc0 - 1u : GS - 1u;
@@ -1255,7 +1440,7 @@ __global__ void __launch_bounds__(256, M::NV <= 8 ? 4 : 1) k_resolve(BatchDev b,
     } else if (tid <= g_last) {
       add_pair(&run_shard(b, s_run[tid])->moves_requests, s_pre[tid + 1] - s_pre[tid], s_dpre[tid + 1] - s_dpre[tid]);
     }
-    for (uint32_t e = tid; e < total; e += blockDim.x) {
+    for (uint32_t e = tid; e < to_move; e += blockDim.x) {
       uint32_t lo = 0, hi = GS;  // the sub-chunk j with s_pre[j] <= e < s_pre[j+1]
       while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
@@ -1276,21 +1461,7 @@ __global__ void __launch_bounds__(256, M::NV <= 8 ? 4 : 1) k_resolve(BatchDev b,
       const uint32_t step = rs->step;
       const MapDev& mp = maps[rd.map_base + (step / rd.steps_per_map) % rd.n_maps];
       const U4 u = draw4(rd.seed, slot, step, TAG_TRANSPORT, 0u);
-      const uint32_t m = mp.m;
-      if (mp.move_row) {  // the compartment's 64-byte record: 5 cdf columns, 6 neighbours
-        const GLOBAL_AS u32x4* rw = (const GLOBAL_AS u32x4*)(gp(mp.move_row) + (size_t)pos * 16);
-        const u32x4 q0 = rw[0], q1 = rw[1], q2 = rw[2], q3 = rw[3];
-        const double uy = u01(u.y);
-        const uint32_t col = (uy > __hiloint2double((int)q0.y, (int)q0.x) ? 1u : 0u) +
-                             (uy > __hiloint2double((int)q0.w, (int)q0.z) ? 1u : 0u) +
-                             (uy > __hiloint2double((int)q1.y, (int)q1.x) ? 1u : 0u) +
-                             (uy > __hiloint2double((int)q1.w, (int)q1.z) ? 1u : 0u) +
-                             (uy > __hiloint2double((int)q2.y, (int)q2.x) ? 1u : 0u);
-        pos = col == 0 ? q2.z : col == 1 ? q2.w : col == 2 ? q3.x : col == 3 ? q3.y : col == 4 ? q3.z : q3.w;
-      } else {
-        const uint32_t col = cdf_column(gp(mp.cdf) + (size_t)pos * m, m, u01(u.y));
-        pos = gp(mp.nbr)[(size_t)pos * m + col];
-      }
+      pos = next_place(mp, pos, u01(u.y));
       b.pos[g] = pos;
       bool exits = false;
       if (rd.enable_leave && leave_stage && !(ms & MOVER_INACTIVE)) {
@@ -1602,8 +1773,26 @@ static const void* kernel_ptr_lv(int blk, bool priv, bool win) {
   if (blk == 1024) return (const void*)&k_particle<M, 1024, M::NL, lane_interleave(M::NL), true, false, false, LV>;
   return nullptr;
 }
+template <class M, bool LV>
+static const void* small_ptr(int blk) {
+  return blk == 256   ? (const void*)&k_particle_small<M, 256, LV>
+         : blk == 512 ? (const void*)&k_particle_small<M, 512, LV>
+                      : (const void*)&k_particle_small<M, 1024, LV>;
+}
+template <class M, bool LV>
+static void launch_small(const BatchDev& b, const ParticleLaunch& L, hipStream_t s) {
+  const uint32_t* off = b.tile_off;
+  const RunState* rs = b.rs;
+  if (L.block == 256)
+    hipLaunchKernelGGL((k_particle_small<M, 256, LV>), dim3(L.grid), dim3(256), L.lds, s, b, b.runs, rs, b.maps, off);
+  else if (L.block == 512)
+    hipLaunchKernelGGL((k_particle_small<M, 512, LV>), dim3(L.grid), dim3(512), L.lds, s, b, b.runs, rs, b.maps, off);
+  else
+    hipLaunchKernelGGL((k_particle_small<M, 1024, LV>), dim3(L.grid), dim3(1024), L.lds, s, b, b.runs, rs, b.maps, off);
+}
 template <class M>
-static const void* kernel_ptr_t(int blk, bool priv, bool probe, bool win, bool leave) {
+static const void* kernel_ptr_t(int blk, bool priv, bool probe, bool win, bool leave, bool small) {
+  if (small) return leave ? small_ptr<M, true>(blk) : small_ptr<M, false>(blk);
   if (probe) {
     if (!priv) return (const void*)&k_particle<M, 256, M::NL, lane_interleave(M::NL), false, true, false, true>;
     return win ? (const void*)&k_particle<M, 256, M::NL, lane_interleave(M::NL), true, true, true, true>
@@ -1637,7 +1826,12 @@ static void launch_lv(const BatchDev& b, const ParticleLaunch& L, hipStream_t s)
 }
 template <class M>
 static void launch_t(const BatchDev& b, const ParticleLaunch& L, hipStream_t s) {
-  if (L.probe) {
+  if (b.moved) {
+    if (L.leave)
+      launch_small<M, true>(b, L, s);
+    else
+      launch_small<M, false>(b, L, s);
+  } else if (L.probe) {
     if (!L.priv)
       launch_particle_t<M, 256, false, true, false, true>(b, L.grid, 0, s);
     else if (L.win)
