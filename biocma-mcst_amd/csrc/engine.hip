@@ -808,11 +808,11 @@ int choose_launch(mcst_engine* e) {
   for (const auto& h : e->runs)
     if (h.phase == 1) entries += (uint64_t)h.n_s * h.n_c;
   b.n_copies = entries <= S_COPY_ENTRIES ? run_copies(M.ns) : 1u;
-  e->grid_aux = (int)std::min<uint64_t>(((uint64_t)b.n_comp_total + 255) / 256, 8192);
+  e->grid_aux = (int)std::min<uint64_t>(((uint64_t)b.n_chunk_total + 3) / 4, 8192);
   e->plaunch = best;
   e->grid_particle = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)prop.multiProcessorCount * 4, b.T_max));
   // one thread per compartment, plus the block that lays out the tiles
-  e->grid_transport = (int)std::min<uint64_t>(((uint64_t)b.n_comp_total + 255) / 256, 8192) + 1;
+  e->grid_transport = (int)std::min<uint64_t>(((uint64_t)b.n_chunk_total + 3) / 4, 8192) + 1;
   // resolve: enough blocks for groups of 32 sub-chunks, up to the blocks
   // that are resident at once (a second round of blocks would start after
   // the first had worked through their groups); the kernel picks 32 or 64
@@ -838,7 +838,7 @@ int refresh_tables(mcst_engine* e) {
   uint32_t n_comp = 0;
   for (uint32_t r = 0; r < R; ++r) {
     e->comp_off[r] = n_comp;
-    if (e->runs[r].phase == 1) n_comp += e->runs[r].n_c;
+    if (e->runs[r].phase == 1) n_comp += (e->runs[r].n_c + 63) / 64;
   }
   e->comp_off[R] = n_comp;
   HIP_TRY(hipMemcpy(e->d_comp, e->comp_off.data(), (R + 1) * sizeof(uint32_t), hipMemcpyHostToDevice));
@@ -853,7 +853,7 @@ int refresh_tables(mcst_engine* e) {
   if (!e->h_maps.empty())
     HIP_TRY(hipMemcpy(e->d_maps, e->h_maps.data(), e->h_maps.size() * sizeof(MapDev), hipMemcpyHostToDevice));
   b.R = R;
-  b.n_comp_total = n_comp;
+  b.n_chunk_total = n_comp;
   b.maps = e->d_maps;
   e->any_leave = false;
   e->max_tiles = 0;
@@ -1155,7 +1155,7 @@ int commit(mcst_engine* e) {
   b.P = P;
   b.T_max = (uint32_t)T_max;
   b.R = 0;
-  b.n_comp_total = 0;
+  b.n_chunk_total = 0;
   // lists sized for the particle pass with the most sub-chunks per tile that
   // the pool may use (choose_launch)
   b.nsub = list_subs(M, T_max);

@@ -268,10 +268,10 @@ struct BatchDev {
   RunState* rs;
   RunShard* shards;         // [R][n_shard]
   const MapDev* maps;
-  const uint32_t* comp_off; // [R+1]
+  const uint32_t* comp_off; // [R+1] 64-compartment chunks before each run (none of a run off the device)
   uint32_t R;
   uint32_t n_shard;
-  uint32_t n_comp_total;
+  uint32_t n_chunk_total;
   uint32_t ns_max;          // largest species count of the batch
   uint32_t T_max;
   uint32_t nsub;            // sub-chunks per tile of the particle pass in use

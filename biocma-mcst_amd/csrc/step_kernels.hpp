@@ -95,39 +95,65 @@ template <uint32_t NT>
 __device__ void layout_pass(const BatchDev& b);
 
 // sum_i C[s][i] * M(i, j) over column j of a transport matrix stored by
-// destination column, for every species: entries in groups of 8 whose loads
-// are all in flight together (a column holds the degree plus the diagonal,
-// rarely more than 8); the sums still run in entry order.
+// destination column, for every species, in entry order.  The transport is a
+// chain of dependent loads on the critical path of a step, so it is cut where
+// it can be: start() requests the first group of entries before the caller's
+// other loads, and finish() requests each next group with the concentrations of
+// the one before (a column holds the degree plus the diagonal, mostly 7 or 8).
+// With the terms beside the inflow loaded before it and scalar run fields, the
+// resolve kernel of 345 679 particles in 777 compartments takes 9.0 us instead
+// of 10.1, of 250 003 in 1989 of 4 species 9.9 instead of 13.2.
 template <int NS>
-__device__ __forceinline__ void column_inflow(const GLOBAL_AS uint32_t* col_ptr, const GLOBAL_AS uint32_t* src,
-                                              const GLOBAL_AS double* val, const GLOBAL_AS double* c, uint32_t n_c,
-                                              uint32_t j, double (&acc)[NS]) {
-#pragma unroll
-  for (int s = 0; s < NS; ++s) acc[s] = 0.0;
-  const uint32_t e0 = col_ptr[j], e1 = col_ptr[j + 1];
-  constexpr uint32_t EG = NS >= 2 ? 4u : 8u;  // entries in flight: fewer for many species (registers)
-  for (uint32_t e = e0; e < e1; e += EG) {
-    uint32_t i[EG];
-    double v[EG], cv[EG][NS];
+struct ColumnInflow {
+  static constexpr uint32_t EG = NS >= 4 ? 2u : 4u;  // entries in a group: fewer for many species (registers)
+  const GLOBAL_AS uint32_t* src;
+  const GLOBAL_AS double* val;
+  uint32_t e, e1;
+  uint32_t i[EG];
+  double v[EG];
+  __device__ __forceinline__ void request(uint32_t (&ni)[EG], double (&nv)[EG], uint32_t from) const {
 #pragma unroll
     for (uint32_t k = 0; k < EG; ++k) {
-      const uint32_t ek = e + k < e1 ? e + k : e1 - 1u;
-      i[k] = src[ek];
-      v[k] = val[ek];
+      const uint32_t ek = from + k < e1 ? from + k : e1 - 1u;
+      ni[k] = src[ek];
+      nv[k] = val[ek];
     }
-#pragma unroll
-    for (uint32_t k = 0; k < EG; ++k)
-#pragma unroll
-      for (int s = 0; s < NS; ++s) cv[k][s] = c[(size_t)s * n_c + i[k]];
-#pragma unroll
-    for (uint32_t k = 0; k < EG; ++k)
-      if (e + k < e1)
-#pragma unroll
-        for (int s = 0; s < NS; ++s) acc[s] += cv[k][s] * v[k];
   }
-}
+  __device__ __forceinline__ void start(const uint32_t* col_ptr, const uint32_t* s, const double* w, uint32_t j) {
+    e = gp(col_ptr)[j];
+    e1 = gp(col_ptr)[j + 1];
+    src = gp(s);
+    val = gp(w);
+    if (e < e1) request(i, v, e);
+  }
+  __device__ __forceinline__ void finish(const GLOBAL_AS double* c, uint32_t n_c, double (&acc)[NS]) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[s] = 0.0;
+    while (e < e1) {
+      double cv[EG][NS];
+#pragma unroll
+      for (uint32_t k = 0; k < EG; ++k)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) cv[k][s] = c[(size_t)s * n_c + i[k]];
+      uint32_t ni[EG];
+      double nv[EG];
+      if (e + EG < e1) request(ni, nv, e + EG);
+#pragma unroll
+      for (uint32_t k = 0; k < EG; ++k)
+        if (e + k < e1)
+#pragma unroll
+          for (int s = 0; s < NS; ++s) acc[s] += cv[k][s] * v[k];
+#pragma unroll
+      for (uint32_t k = 0; k < EG; ++k) {
+        i[k] = ni[k];
+        v[k] = nv[k];
+      }
+      e += EG;
+    }
+  }
+};
 
-// The transport of batch compartment g for the step `ahead` steps after its
+// The transport of compartment j of run r for the step `ahead` steps after its
 // run's current one (0: the step about to run; 1: the next one, computed
 // during this step's resolve kernel).  It reads C and the contributions of
 // the last pass, from S or (TAKE > 0) from the TAKE accumulators the pass has
@@ -145,17 +171,15 @@ __device__ __forceinline__ void column_inflow(const GLOBAL_AS uint32_t* col_ptr,
 // fields again, a round trip each).
 template <class M, int TAKE>
 __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* __restrict__ runs,
-                                              const MapDev* __restrict__ maps, uint32_t g, uint32_t ahead) {
+                                              const MapDev* __restrict__ maps, uint32_t r, uint32_t j, uint32_t ahead) {
   constexpr int NS = M::NS;
   constexpr int NR = record_terms<M>();
   constexpr uint32_t KM = TAKE ? (uint32_t)TAKE : 1u;
-  const uint32_t r = find_run(b.comp_off, b.R, g);
   const RunDev& rd = runs[r];
   // the step being prepared; the run's activity is recomputed here rather
   // than read from the layout, which other blocks write concurrently
   const uint32_t step = b.rs[r].step + ahead;
   if (step - ahead >= rd.step_target) return;  // the run did not take (or does not take) this step
-  const uint32_t j = g - b.comp_off[r];
   const uint32_t n_c = rd.n_c;
   // the contributions of the last pass
   double sp[KM][NS];
@@ -184,24 +208,28 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
     return;
   }
   const MapDev& mp = maps[rd.map_base + (step / rd.steps_per_map) % rd.n_maps];
+  const bool flow = (b.stages & STAGE_TRANSPORT) != 0;
+  ColumnInflow<NS> in;
+  if (flow) in.start(mp.col_ptr, mp.src, mp.val, j);
+  const GLOBAL_AS double* c = gp(rd.C[step & 1u]);
+  double cn[NS], mn[NS];  // new concentrations and masses
+#pragma unroll
+  for (int s = 0; s < NS; ++s) cn[s] = c[(size_t)s * n_c + j];
   const double p_move = gp(mp.p_move)[j];
   double qx = gp(mp.q_exit)[j];
   const double* const vf = rd.vf_q + (size_t)(step % VF_ROWS) * rd.vf_w;  // this step's flows (n_vf > 0)
   if (rd.n_vf && rd.vx_slot[j] >= 0) qx = vf[rd.n_vf + (uint32_t)rd.vx_slot[j]];
-  const GLOBAL_AS double* c = gp(rd.C[step & 1u]);
   const bool gas = rd.Cg[0] != nullptr;
-  double cn[NS], mn[NS];  // new concentrations and masses
-#pragma unroll
-  for (int s = 0; s < NS; ++s) cn[s] = c[(size_t)s * n_c + j];
-  if (b.stages & STAGE_TRANSPORT) {
-    double acc[NS];
-    column_inflow<NS>(gp(mp.col_ptr), gp(mp.src), gp(mp.val), c, n_c, j, acc);
+  if (flow) {
     double sink = gp(rd.sink)[j];
     const double inv_v = gp(mp.inv_v)[j];
     double fv[NS], fvg[NS];  // time-dependent feeds of this compartment, in feed order
     double sink_g = gas ? gp(rd.sink_g)[j] : 0.0;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) fv[s] = fvg[s] = 0.0;
+    for (int s = 0; s < NS; ++s) {
+      fv[s] = fvg[s] = 0.0;
+      mn[s] = gp(rd.m)[(size_t)s * n_c + j];
+    }
     if (rd.n_vf) {
       for (uint32_t q = rd.vf_sink_ptr[j]; q < rd.vf_sink_ptr[j + 1]; ++q) {
         const uint32_t k = rd.vf_sink_k[q];
@@ -220,6 +248,15 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
         }
       }
     }
+    // the terms beside the inflow
+    double src_f[NS], out[NS], mtr[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      src_f[s] = source(s) + (gp(rd.F)[(size_t)s * n_c + j] + fv[s]);
+      out[s] = cn[s] * sink;
+      mtr[s] = 0.0;
+    }
+    double acc[NS];
     if (gas) {
       // two-phase step (SimulationUnit::ode_step, simulation.model.cpp:131-150):
       // mtr = kla*(H*C_gas - C)*V from the old concentrations, the gas
@@ -227,24 +264,19 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
       // implScalar.cpp:228-248), then clearNegs on the liquid
       // (implScalar.cpp:266-297): a value in (-1e-4*5e-3, 0) becomes 0
       const GLOBAL_AS double* cg = gp(rd.Cg[step & 1u]);
-      double accg[NS];
-      column_inflow<NS>(gp(mp.g_col_ptr), gp(mp.g_src), gp(mp.g_val), cg, n_c, j, accg);
+      ColumnInflow<NS> in_g;
+      in_g.start(mp.g_col_ptr, mp.g_src, mp.g_val, j);
+      in_g.finish(cg, n_c, acc);
       const double inv_vg = gp(mp.g_inv_v)[j];
-      const double tol = 1e-4 * 5e-3;
       double cgn[NS], mgn[NS];
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const size_t o = (size_t)s * n_c + j;
         const double cgs = cg[o];
-        const double mtr = (gp(mp.g_kla)[o] * ((cgs * rd.henry[s]) - cn[s])) * gp(mp.vol)[j];
-        const double dg = ((accg[s] - cgs * sink_g) + (gp(rd.Fg)[o] + fvg[s])) - mtr;
+        mtr[s] = (gp(mp.g_kla)[o] * ((cgs * rd.henry[s]) - cn[s])) * gp(mp.vol)[j];
+        const double dg = ((acc[s] - cgs * sink_g) + (gp(rd.Fg)[o] + fvg[s])) - mtr[s];
         mgn[s] = gp(rd.mg)[o] + rd.dt * dg;
         cgn[s] = mgn[s] * inv_vg;
-        const double dl = ((acc[s] - cn[s] * sink) + (source(s) + (gp(rd.F)[o] + fv[s]))) + mtr;
-        mn[s] = gp(rd.m)[o] + rd.dt * dl;
-        double cl = mn[s] * inv_v;
-        if (cl < 0.0 && fabs(cl) < tol) cl = 0.0;
-        cn[s] = cl;
       }
       GLOBAL_AS double* const Cgn = gp(rd.Cg[(step + 1u) & 1u]) + j;
       GLOBAL_AS double* const mg_out = gp(rd.mg) + j;
@@ -253,16 +285,25 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
         Cgn[(size_t)s * n_c] = cgn[s];
         mg_out[(size_t)s * n_c] = mgn[s];
       }
-    } else {
+    } else if (rd.kla) {  // gas-liquid transfer from a fixed gas phase: kla*(C* - C)*V
+      const double vol = gp(mp.vol)[j];
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const size_t o = (size_t)s * n_c + j;
-        double dmdt = (acc[s] - cn[s] * sink) + (source(s) + (gp(rd.F)[o] + fv[s]));
-        // gas-liquid transfer from a fixed gas phase: kla*(C* - C)*V
-        if (rd.kla) dmdt = dmdt + (gp(rd.kla)[o] * (gp(rd.cstar)[o] - cn[s])) * gp(mp.vol)[j];
-        mn[s] = gp(rd.m)[o] + rd.dt * dmdt;
-        cn[s] = mn[s] * inv_v;
+        mtr[s] = (gp(rd.kla)[o] * (gp(rd.cstar)[o] - cn[s])) * vol;
       }
+    }
+    in.finish(c, n_c, acc);
+    const double tol = 1e-4 * 5e-3;
+    const bool transfer = gas || rd.kla;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      double dmdt = (acc[s] - out[s]) + src_f[s];
+      if (transfer) dmdt = dmdt + mtr[s];
+      mn[s] = mn[s] + rd.dt * dmdt;
+      double cl = mn[s] * inv_v;
+      if (gas && cl < 0.0 && fabs(cl) < tol) cl = 0.0;
+      cn[s] = cl;
     }
   }
   double rt[NR];
@@ -278,7 +319,7 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
   for (int s = 0; s < NS; ++s) {
     const size_t o = (size_t)s * n_c;
     Cn[o] = cn[s];
-    if (b.stages & STAGE_TRANSPORT) m_out[o] = mn[s];
+    if (flow) m_out[o] = mn[s];
   }
   if constexpr (TAKE > 0) clear();
 }
@@ -288,9 +329,14 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
 template <class M, int TAKE>
 __device__ void transport_compartments(const BatchDev& b, const RunDev* __restrict__ runs,
                                        const MapDev* __restrict__ maps, uint32_t blk, uint32_t n_blk, uint32_t ahead) {
-  const uint32_t total = b.n_comp_total;
-  const uint32_t stride = n_blk * blockDim.x;
-  for (uint32_t g = blk * blockDim.x + threadIdx.x; g < total; g += stride) transport_one<M, TAKE>(b, runs, maps, g, ahead);
+  // a wave takes 64 compartments of one run (comp_off counts such chunks), so
+  // that the run's and the flowmap's fields are scalars
+  const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u, wpb = blockDim.x >> 6;
+  for (uint32_t q = blk * wpb + wave; q < b.n_chunk_total; q += n_blk * wpb) {
+    const uint32_t r = find_run(b.comp_off, b.R, q);
+    const uint32_t j = (q - b.comp_off[r]) * 64u + lane;
+    if (j < runs[r].n_c) transport_one<M, TAKE>(b, runs, maps, r, j, ahead);
+  }
 }
 
 template <class M>
