@@ -600,7 +600,7 @@ __global__ void __launch_bounds__(BLK)
         st |= (uint32_t)ld_stream(gp(b.status) + ij) << (8 * j);
         a.pos[j] = ld_stream(gp(b.pos) + ij);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) a.x[v][j] = ld_stream(gp(b.state) + (uint64_t)v * P + ij);
+        for (int v = 0; v < NV; ++v) a.x[v][j] = reads_var<M>(v) ? ld_stream(gp(b.state) + (uint64_t)v * P + ij) : 0.0;
       }
       a.st = st;
     } else {
@@ -608,7 +608,12 @@ __global__ void __launch_bounds__(BLK)
       a.st = ld_lane<NL>(gp(b.status) + i0);
       ld_lane<NL>(gp(b.pos) + i0, a.pos);
 #pragma unroll
-      for (int v = 0; v < NV; ++v) ld_lane<NL>(gp(b.state) + (uint64_t)v * P + i0, a.x[v]);
+      for (int v = 0; v < NV; ++v) {
+        if (reads_var<M>(v))
+          ld_lane<NL>(gp(b.state) + (uint64_t)v * P + i0, a.x[v]);
+        else
+          for (int j = 0; j < NL; ++j) a.x[v][j] = 0.0;
+      }
     }
   };
   auto gather = [&](const SubRef& q, const Sub& a, double (&rr)[NL][NQ]) {
@@ -669,7 +674,8 @@ __global__ void __launch_bounds__(BLK)
   for (int j = 0; j < NL; ++j) {
     asm volatile("" : "+v"(A.pos[j]));
 #pragma unroll
-    for (int v = 0; v < NV; ++v) asm volatile("" : "+v"(A.x[v][j]));
+    for (int v = 0; v < NV; ++v)
+      if (reads_var<M>(v)) asm volatile("" : "+v"(A.x[v][j]));
 #pragma unroll
     for (int f = 0; f < NQ; ++f) asm volatile("" : "+v"(rr[j][f]));
   }
@@ -758,7 +764,7 @@ __global__ void __launch_bounds__(BLK)
     // ---- per-particle work: arithmetic only
     const uint32_t i0 = NL * lane;  // contiguous layout: sub-chunk-relative slot of j = 0
     const bool pair_valid = i0 < cur.cnt;
-    bool valid[NL], idle[NL], want[NL], mover[NL], exited[NL], dead[NL];
+    bool valid[NL], idle[NL], updated[NL], want[NL], mover[NL], exited[NL], dead[NL];
     double x[NL][NV];
     double contrib[NL][NS];
 #pragma unroll
@@ -766,6 +772,7 @@ __global__ void __launch_bounds__(BLK)
       const uint32_t stj = (A.st >> (8 * j)) & 0xFFu;
       valid[j] = off(j) < cur.cnt;
       idle[j] = valid[j] && stj == IDLE;
+      updated[j] = idle[j] && do_model;  // its state changes
       want[j] = mover[j] = exited[j] = dead[j] = false;
 #pragma unroll
       for (int v = 0; v < NV; ++v) x[j][v] = A.x[v][j];
@@ -884,10 +891,17 @@ __global__ void __launch_bounds__(BLK)
       for (int j = 0; j < NL; ++j) {
         if (!(want[j] && rd_[j] < DIV_STAGE)) continue;
         GLOBAL_AS double* stg = gp(b.div_stage) + ((uint64_t)sc * DIV_STAGE + rd_[j]) * NV;
+        GLOBAL_AS double* const sj = gp(b.state) + cur.base + off(j);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) stg[v] = x[j][v];
+        for (int v = 0; v < NV; ++v) {
+          if (!reads_var<M>(v) && !writes_var<M>(v)) x[j][v] = sj[(uint64_t)v * P];
+          stg[v] = x[j][v];
+        }
         double xd[NV];
         M::division(p, x[j], xd, RngKey{seed, cur.slot0 + off(j), step});
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+          if (!writes_var<M>(v)) sj[(uint64_t)v * P] = x[j][v];
       }
     }
 
@@ -897,19 +911,38 @@ __global__ void __launch_bounds__(BLK)
     if constexpr (ILV) {
 #pragma unroll
       for (int j = 0; j < NL; ++j) {
-        if (!valid[j]) continue;
+        if (!updated[j]) continue;
         const uint64_t gj = cur.base + off(j);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) st_stream(gp(b.state) + (uint64_t)v * P + gj, x[j][v]);
+        for (int v = 0; v < NV; ++v)
+          if (writes_var<M>(v)) st_stream(gp(b.state) + (uint64_t)v * P + gj, x[j][v]);
+      }
+#pragma unroll
+      for (int j = 0; j < NL; ++j) {
+        const uint64_t gj = cur.base + off(j);
         if (exited[j] || dead[j]) gp(b.status)[gj] = dead[j] ? (uint8_t)DEAD : (uint8_t)EXIT;
       }
     } else {
+      bool all = true;
 #pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        double xv[NL];
+      for (int j = 0; j < NL; ++j) all = all && updated[j];
+      if (all) {
 #pragma unroll
-        for (int j = 0; j < NL; ++j) xv[j] = x[j][v];
-        if (pair_valid) st_lane<NL>(gp(b.state) + (uint64_t)v * P + gi, xv);
+        for (int v = 0; v < NV; ++v) {
+          if (!writes_var<M>(v)) continue;
+          double xv[NL];
+#pragma unroll
+          for (int j = 0; j < NL; ++j) xv[j] = x[j][v];
+          st_lane<NL>(gp(b.state) + (uint64_t)v * P + gi, xv);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+          if (!updated[j]) continue;
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+            if (writes_var<M>(v)) st_stream(gp(b.state) + (uint64_t)v * P + gi + (uint32_t)j, x[j][v]);
+        }
       }
       uint32_t stn = A.st;
       bool changed = false;
@@ -1043,7 +1076,8 @@ __global__ void __launch_bounds__(BLK)
       st = gp(b.status)[g];
       pos = gp(b.pos)[g];
 #pragma unroll
-      for (int v = 0; v < NV; ++v) x[v] = gp(b.state)[(uint64_t)v * P + g];
+      for (int v = 0; v < NV; ++v)
+        if (reads_var<M>(v)) x[v] = gp(b.state)[(uint64_t)v * P + g];
     }
     // ---- block-uniform: the run whose contributions the LDS accumulates
     const uint32_t r0 = find_run(tile_off, R, (grp * WPB) / NSUB);
@@ -1113,10 +1147,17 @@ __global__ void __launch_bounds__(BLK)
       if (want) {
         if (rk < DIV_STAGE) {
           GLOBAL_AS double* stg = gp(b.div_stage) + ((uint64_t)sc * DIV_STAGE + rk) * NV;
+          GLOBAL_AS double* const sg = gp(b.state) + g;
 #pragma unroll
-          for (int v = 0; v < NV; ++v) stg[v] = x[v];
+          for (int v = 0; v < NV; ++v) {
+            if (!reads_var<M>(v) && !writes_var<M>(v)) x[v] = sg[(uint64_t)v * P];
+            stg[v] = x[v];
+          }
           double xd[NV];
           M::division(p, x, xd, RngKey{rd.seed, slot, step});
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+            if (!writes_var<M>(v)) sg[(uint64_t)v * P] = x[v];
         }
         const uint32_t pv = pos < LIST_POS_FAR ? pos : LIST_POS_FAR;
         gp(b.div_rec)[seg + rk] = (slot % TILE) | (pv << LIST_POS_SHIFT);
@@ -1126,9 +1167,10 @@ __global__ void __launch_bounds__(BLK)
       if (lane < 2) atomicAdd((lane ? b.div_l2 : b.div_l1) + (sc >> (lane ? 12 : 6)), n_div);
     }
     // ---- stores
-    if (valid) {
+    if (idle && do_model) {
 #pragma unroll
-      for (int v = 0; v < NV; ++v) gp(b.state)[(uint64_t)v * P + g] = x[v];
+      for (int v = 0; v < NV; ++v)
+        if (writes_var<M>(v)) gp(b.state)[(uint64_t)v * P + g] = x[v];
     }
     if (mover) gp(b.pos)[g] = to;
     if (exited || dead) {
