@@ -477,6 +477,7 @@ struct mcst_engine {
   uint32_t* alt_clk_hyd = nullptr;
   uint32_t* alt_clk_div = nullptr;
   uint64_t alt_P = 0;
+  uint32_t layout = 0;              // which of the two tile tables the step under way reads (launch_step)
   int grid_aux = 1;                 // the resolve kernel's blocks that take the contributions
   int tuned_group = -1;
   int grid_move = 1;
@@ -1174,6 +1175,7 @@ int commit(mcst_engine* e) {
   if ((rc = dev_alloc(e, (void**)&b.tile_cnt, T_max * sizeof(unsigned long long)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.tile_pre, (T_max + 1) * sizeof(unsigned long long)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.tile_off, (RC + 1) * sizeof(uint32_t)))) return rc;
+  if ((rc = dev_alloc(e, (void**)&b.tile_off_next, (RC + 1) * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.move_rec, T_max * TILE * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.div_rec, T_max * TILE * sizeof(uint32_t)))) return rc;
   if ((rc = dev_alloc(e, (void**)&b.div_pos, T_max * TILE * sizeof(uint32_t)))) return rc;
@@ -1197,6 +1199,7 @@ int commit(mcst_engine* e) {
   HIP_TRY(hipMemset(b.ticket, 0, (2 + RESOLVE_TICKETS) * TICKET_STRIDE * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.rm_tile_off, 0, (RC + 1) * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.tile_off, 0, (RC + 1) * sizeof(uint32_t)));
+  HIP_TRY(hipMemset(b.tile_off_next, 0, (RC + 1) * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.sub_moves, 0, T_max * b.nsub * sizeof(uint32_t)));
   HIP_TRY(hipMemset(b.sub_divs, 0, T_max * b.nsub * sizeof(uint32_t)));
   HIP_TRY(hipMemset(e->d_rs, 0, (size_t)RC * sizeof(RunState)));
@@ -1251,6 +1254,11 @@ void launch_step(mcst_engine* e, uint32_t stages, const hipEvent_t* ev = nullptr
                  bool ahead = false) {
   if (e->bd.R == 0) return;  // no run admitted yet
   BatchDev b = e->bd;
+  // k_transport lays out a step's tiles in the first table; a step whose
+  // resolve kernel transports the next one lays that one out in the other
+  if (!transported) e->layout = 0;
+  if (e->layout) std::swap(b.tile_off, b.tile_off_next);
+  if (ahead) e->layout ^= 1u;
   b.stages = stages;
   const uint32_t nv = (uint32_t)e->model->nv;
   const ModelOps& ops = *e->model->ops;

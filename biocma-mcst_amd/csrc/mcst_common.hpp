@@ -251,7 +251,8 @@ struct BatchDev {
   // per-tile bookkeeping of the removal
   unsigned long long* tile_cnt;  // [T_max] gaps (low 32 bits) and fillers (high) of each tile
   unsigned long long* tile_pre;  // [T_max+1] their sums before each tile
-  uint32_t* tile_off;       // [R+1] first global tile of each run in the current layout
+  uint32_t* tile_off;       // [R+1] first global tile of each run in the step's layout
+  uint32_t* tile_off_next;  // the next step's, written by the books while blocks of the step may yet read tile_off
   // lists of the particle pass, one segment of TILE/nsub entries per sub-chunk
   uint32_t* move_rec;       // [T_max*TILE] particles leaving their compartment, one entry each
                             // (slot, flag and compartment in one word, so that the few movers of a

@@ -1192,14 +1192,6 @@ __global__ void __launch_bounds__(BLK)
   flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
 }
 
-// The books of every run after its step, kept by the last block of
-// k_resolve: counters, births (the accepted requests), the removal decision
-// of update_and_remove_inactive (particles_container.hpp:539-557, threshold
-// from the pass's count) over [0, n_end) where the newborns already sit, and
-// the removal's tile layout; then the request block counts are cleared for
-// the next pass (n_sc: the sub-chunks of this step's layout).  With `layout`
-// it also lays out the next step's tiles (layout_pass), from the counts it
-// has just computed.
 // What the books read of a run, requested together (before its counter shards
 // are, so that both round trips to memory overlap).
 struct RunBooks {
@@ -1290,6 +1282,16 @@ __device__ __forceinline__ void keep_books(const BatchDev& b, RunState* rs, RunB
   }
 }
 
+// The books of every run after its step, kept by the last block of
+// k_resolve: counters, births (the accepted requests), the removal decision
+// of update_and_remove_inactive (particles_container.hpp:539-557, threshold
+// from the pass's count) over [0, n_end) where the newborns already sit, and
+// the removal's tile layout; then the request block counts are cleared for
+// the next pass (n_sc: the sub-chunks of this step's layout).  With `layout`
+// it also lays out the next step's tiles (layout_pass), from the counts it
+// has just computed, in the other of two tables: a resolve block without a
+// group is not waited for, so it may start after the books and must still find
+// the step's own tile count, or it would take itself for a block with work.
 __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs, uint32_t n_sc, bool layout) {
   constexpr uint32_t NT = 256, NWV = NT / 64;
   __shared__ uint32_t s_w[NWV], s_wl[NWV];
@@ -1323,8 +1325,8 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
         b.rm_tile_off[0] = 0u;
         b.rm_tile_off[1] = tiles;
         if (layout) {
-          b.tile_off[0] = 0u;
-          b.tile_off[1] = tiles_l;
+          b.tile_off_next[0] = 0u;
+          b.tile_off_next[1] = tiles_l;
           b.rs[0].tile_begin = 0u;
         }
       }
@@ -1368,7 +1370,7 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
       if (r < b.R) {
         b.rm_tile_off[r] = carry + wpre + inc - tiles;
         if (layout) {
-          b.tile_off[r] = carry_l + wpre_l + inc_l - tiles_l;
+          b.tile_off_next[r] = carry_l + wpre_l + inc_l - tiles_l;
           b.rs[r].tile_begin = carry_l + wpre_l + inc_l - tiles_l;
         }
       }
@@ -1381,7 +1383,7 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
     }
     if (tid == 0) {
       b.rm_tile_off[b.R] = s_carry;
-      if (layout) b.tile_off[b.R] = s_carry_l;
+      if (layout) b.tile_off_next[b.R] = s_carry_l;
     }
   }
   for (uint32_t i = tid; i < (n_sc + 63u) >> 6; i += NT) b.div_l1[i] = 0u;

@@ -15,7 +15,7 @@
 
 namespace mcst {
 
-constexpr uint32_t UDF_ABI_VERSION = 16;
+constexpr uint32_t UDF_ABI_VERSION = 17;
 
 struct UdfModel {
   uint32_t abi_version;
