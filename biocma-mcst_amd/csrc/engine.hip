@@ -478,6 +478,8 @@ struct mcst_engine {
   uint32_t* alt_clk_div = nullptr;
   uint64_t alt_P = 0;
   uint32_t layout = 0;              // which of the two tile tables the step under way reads (launch_step)
+  double* part_mem = nullptr;       // contribution rows of the particle pass (BatchDev::part), part_bytes allocated
+  size_t part_bytes = 0;
   int grid_aux = 1;                 // the resolve kernel's blocks that take the contributions
   int tuned_group = -1;
   int grid_move = 1;
@@ -540,6 +542,8 @@ void drop_graph(mcst_engine* e) {
 
 void release(mcst_engine* e) {
   drop_graph(e);
+  e->part_mem = nullptr;  // freed with allocs
+  e->part_bytes = 0;
   e->alt_pos = nullptr;  // freed with allocs
   e->alt_status = nullptr;
   e->alt_state = e->alt_age_hyd = e->alt_age_div = nullptr;
@@ -684,7 +688,8 @@ int check_definable(const mcst_engine* e, const HostRun& h, uint32_t r) {
 // Launch shapes for the runs on the device: LDS contribution accumulator
 // when the largest live run's [n_s][n_c] fits, then the block size with the
 // most resident waves, up to 8 per CU; a grid of that many blocks per CU.  MCST_PARTICLE_BLOCK
-// (256/512/1024), MCST_CONTRIB_LDS (0/1) and MCST_TILE_GROUP override.
+// (256/512/1024), MCST_CONTRIB_LDS (0/1), MCST_TILE_GROUP and
+// MCST_CONTRIB_ROWS (0/1) override.
 int choose_launch(mcst_engine* e) {
   const ModelEntry& M = *e->model;
   BatchDev& b = e->bd;
@@ -809,7 +814,38 @@ int choose_launch(mcst_engine* e) {
   for (const auto& h : e->runs)
     if (h.phase == 1) entries += (uint64_t)h.n_s * h.n_c;
   b.n_copies = entries <= S_COPY_ENTRIES ? run_copies(M.ns) : 1u;
-  e->grid_aux = (int)std::min<uint64_t>(((uint64_t)b.n_chunk_total + 3) / 4, 8192);
+  // contribution rows (MCST_CONTRIB_ROWS=1; one live run whose whole
+  // accumulator is in LDS): each block of the pass stores its accumulator as
+  // a row and the resolve kernel sums the rows in a fixed order, instead of
+  // each block adding its accumulator to a copy with FP64 atomics.  Pass and
+  // resolve kernel of 1e7 particles in 5000 compartments (512 rows) 115 and
+  // 21.8 us against 116 and 20.1, of 1e5 in 64 (391 rows) 4.8 and 16.0 against
+  // 5.0 and 6.6: the atomics stay the default.
+  b.part = nullptr;
+  b.part_rows = b.part_w = 0;
+  const char* rows = std::getenv("MCST_CONTRIB_ROWS");
+  if (rows && std::atoi(rows) != 0 && live == 1 && best.priv && !best.win) {
+    const size_t bytes = (size_t)best.grid * entries * sizeof(double);
+    if (bytes > e->part_bytes) {  // a larger row buffer
+      HIP_TRY(hipStreamSynchronize(e->stream));
+      drop_graph(e);
+      if (e->part_mem) {
+        (void)hipFree(e->part_mem);
+        e->allocs.erase(std::remove(e->allocs.begin(), e->allocs.end(), (void*)e->part_mem), e->allocs.end());
+        e->part_mem = nullptr;
+        e->part_bytes = 0;
+      }
+      if (dev_alloc(e, (void**)&e->part_mem, bytes) == MCST_OK) e->part_bytes = bytes;
+    }
+    if (e->part_mem && bytes <= e->part_bytes) {
+      b.part = e->part_mem;
+      b.part_rows = (uint32_t)best.grid;
+      b.part_w = (uint32_t)entries;
+      b.n_copies = 1;
+    }
+  }
+  const uint32_t chunks_per_block = b.part ? 1 : 4;
+  e->grid_aux = (int)std::min<uint64_t>(((uint64_t)b.n_chunk_total + chunks_per_block - 1) / chunks_per_block, 8192);
   e->plaunch = best;
   e->grid_particle = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)prop.multiProcessorCount * 4, b.T_max));
   // one thread per compartment, plus the block that lays out the tiles
@@ -819,14 +855,14 @@ int choose_launch(mcst_engine* e) {
   // the first had worked through their groups); the kernel picks 32 or 64
   // from the step's tile count
   int res_per_cu = 0;
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&res_per_cu, M.ops->resolve_kernel(b.n_copies), 256, 0));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&res_per_cu, M.ops->resolve_kernel(b), 256, 0));
   const uint64_t resident = (uint64_t)prop.multiProcessorCount * (uint64_t)std::max(1, res_per_cu);
   const uint64_t n_sc = (uint64_t)b.T_max * b.nsub;
   e->grid_move = (int)std::max<uint64_t>(1, std::min<uint64_t>(resident, (n_sc + 31) / 32));
   if (std::getenv("MCST_VERBOSE"))
-    std::fprintf(stderr, "[mcst] particle pass: block=%d grid=%d lds=%zu priv=%d group=%u window=%u leave=%d copies=%u (lds cap %zu)\n",
+    std::fprintf(stderr, "[mcst] particle pass: block=%d grid=%d lds=%zu priv=%d group=%u window=%u leave=%d copies=%u rows=%u (lds cap %zu)\n",
                  best.block, best.grid, best.lds, (int)best.priv, b.tile_group, b.acc_w, (int)best.leave,
-                 b.n_copies, lds_cap);
+                 b.n_copies, b.part_rows, lds_cap);
   return MCST_OK;
 }
 

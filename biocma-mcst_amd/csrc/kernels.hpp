@@ -37,7 +37,7 @@ struct ModelOps {
   // resolve: grid blocks plus aux blocks first in the grid, which take the
   // pass's contributions, for the next step's transport (ahead) or into S
   void (*resolve)(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s);
-  const void* (*resolve_kernel)(uint32_t copies);  // for occupancy queries (BatchDev::n_copies)
+  const void* (*resolve_kernel)(const BatchDev& b);  // for occupancy queries (the variant resolve would launch)
   void (*properties)(const BatchDev& b, uint32_t run, uint64_t n, uint32_t n_c, double* values, double* spatial,
                      hipStream_t s);
 };

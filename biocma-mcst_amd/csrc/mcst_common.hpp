@@ -284,6 +284,13 @@ struct BatchDev {
   // k of the particle pass adds to copy k % n_copies, and the resolve kernel
   // sums the copies
   uint32_t n_copies;
+  // contribution rows (one live run whose whole [n_s][n_c] accumulator fits
+  // LDS): block k of the particle pass stores its accumulator at
+  // part[k * part_w], part_w = n_s * n_c, and the resolve kernel sums the
+  // part_rows rows in a fixed order; null: the copies above
+  double* part;
+  uint32_t part_rows;
+  uint32_t part_w;
 };
 
 // A pass ends with every block adding its LDS accumulator to the run's, a

@@ -164,17 +164,20 @@ struct ColumnInflow {
 // sum by shuffles before that chain cost the resolve kernel 2 us).  TAKE
 // without a next step of this call or of the run (`ahead` 0, or the run's step
 // target): the sums go to S, so that S holds the step's contributions
-// whenever the host can read it.
+// whenever the host can read it.  TAKE_ROWS: the contributions are `given`,
+// summed from the rows by the caller.
 //
 // Every load comes before the first store (the arrays may alias as far as the
 // compiler knows: a store in between made it read the run's and the flowmap's
 // fields again, a round trip each).
+constexpr int TAKE_ROWS = -1;
 template <class M, int TAKE>
 __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* __restrict__ runs,
-                                              const MapDev* __restrict__ maps, uint32_t r, uint32_t j, uint32_t ahead) {
+                                              const MapDev* __restrict__ maps, uint32_t r, uint32_t j, uint32_t ahead,
+                                              const double* given = nullptr) {
   constexpr int NS = M::NS;
   constexpr int NR = record_terms<M>();
-  constexpr uint32_t KM = TAKE ? (uint32_t)TAKE : 1u;
+  constexpr uint32_t KM = TAKE > 0 ? (uint32_t)TAKE : 1u;
   const RunDev& rd = runs[r];
   // the step being prepared; the run's activity is recomputed here rather
   // than read from the layout, which other blocks write concurrently
@@ -187,7 +190,7 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
 #pragma unroll
   for (uint32_t k = 0; k < KM; ++k)
 #pragma unroll
-    for (int s = 0; s < NS; ++s) sp[k][s] = from[((size_t)k * NS + s) * n_c];
+    for (int s = 0; s < NS; ++s) sp[k][s] = TAKE == TAKE_ROWS ? given[s] : from[((size_t)k * NS + s) * n_c];
   auto source = [&](int s) -> double {
     double t = sp[0][s];
 #pragma unroll
@@ -195,6 +198,7 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
     return t;
   };
   auto clear = [&]() {
+    if constexpr (TAKE <= 0) return;
 #pragma unroll
     for (uint32_t k = 0; k < KM; ++k)
 #pragma unroll
@@ -321,7 +325,7 @@ __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* _
     Cn[o] = cn[s];
     if (flow) m_out[o] = mn[s];
   }
-  if constexpr (TAKE > 0) clear();
+  clear();
 }
 
 // The transport (or, TAKE, what becomes of the pass's contributions) of every
@@ -336,6 +340,44 @@ __device__ void transport_compartments(const BatchDev& b, const RunDev* __restri
     const uint32_t r = find_run(b.comp_off, b.R, q);
     const uint32_t j = (q - b.comp_off[r]) * 64u + lane;
     if (j < runs[r].n_c) transport_one<M, TAKE>(b, runs, maps, r, j, ahead);
+  }
+}
+
+// With contribution rows: as transport_compartments, a block taking 64
+// compartments.  Each of its waves sums a quarter of the rows, 8 in flight, and the
+// first adds the waves' sums in turn: the order is the rows' alone.
+template <class M>
+__device__ void sum_rows(const BatchDev& b, const RunDev* __restrict__ runs, const MapDev* __restrict__ maps,
+                         uint32_t blk, uint32_t n_blk, uint32_t ahead) {
+  constexpr int NS = M::NS;
+  constexpr uint32_t NWV = 256 / 64;
+  __shared__ double s_sum[NWV][NS][64];
+  const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  for (uint32_t q = blk; q < b.n_chunk_total; q += n_blk) {
+    const uint32_t r = find_run(b.comp_off, b.R, q);
+    const uint32_t n_c = runs[r].n_c, j = (q - b.comp_off[r]) * 64u + lane;
+    if (b.rs[r].step >= runs[r].step_target) continue;  // the run took no step
+    double t[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) t[s] = 0.0;
+    if (j < n_c) {
+      const GLOBAL_AS double* const part = gp(b.part) + j;
+#pragma unroll 8
+      for (uint32_t row = wave; row < b.part_rows; row += NWV)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) t[s] += part[(size_t)row * b.part_w + (size_t)s * n_c];
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) s_sum[wave][s][lane] = t[s];
+    __syncthreads();
+    if (wave == 0 && j < n_c) {
+#pragma unroll
+      for (uint32_t w = 1; w < NWV; ++w)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) t[s] += s_sum[w][s][lane];
+      transport_one<M, TAKE_ROWS>(b, runs, maps, r, j, ahead, t);
+    }
+    __syncthreads();  // read before the next compartments' sums
   }
 }
 
@@ -385,6 +427,14 @@ __device__ __forceinline__ void flush_window(double* s_acc, GLOBAL_AS double* S,
       s_acc[i] = 0.0;
     }
   }
+}
+
+// With contribution rows: the block's row, from its LDS accumulator (null: of
+// a block without slots).
+template <int BLK>
+__device__ __forceinline__ void store_row(const BatchDev& b, const double* s_acc) {
+  GLOBAL_AS double* const row = gp(b.part) + (size_t)blockIdx.x * b.part_w;
+  for (uint32_t i = threadIdx.x; i < b.part_w; i += BLK) row[i] = s_acc ? s_acc[i] : 0.0;
 }
 
 // First column of a cumulative row with cp[c] >= u, clamped to m-1: for a
@@ -548,7 +598,10 @@ __global__ void __launch_bounds__(BLK)
   const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
   const uint32_t G = b.tile_group && b.tile_group < chunk ? b.tile_group : (chunk ? chunk : 1u);
   uint32_t grp = blockIdx.x * G;
-  if (grp >= n_groups) return;  // the whole block
+  if (grp >= n_groups) {  // the whole block
+    if (PRIV && !WIN && b.part) store_row<BLK>(b, nullptr);
+    return;
+  }
   const uint32_t copy = blockIdx.x & (b.n_copies - 1u);  // of each run's accumulator
   auto next_group = [&](uint32_t g) -> uint32_t {
     const uint32_t g0 = g - g % G;
@@ -1013,7 +1066,10 @@ __global__ void __launch_bounds__(BLK)
   }
   if (PRIV) {
     __syncthreads();
-    flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
+    if (!WIN && b.part)
+      store_row<BLK>(b, s_acc);
+    else
+      flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
   }
   flush_counts();
 #pragma unroll
@@ -1049,7 +1105,10 @@ __global__ void __launch_bounds__(BLK)
   const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
   const uint32_t g_first = R == 1 ? blockIdx.x : blockIdx.x * chunk, g_step = R == 1 ? gridDim.x : 1u;
   const uint32_t g_end = R == 1 || n_groups - g_first < chunk ? n_groups : g_first + chunk;
-  if (g_first >= n_groups) return;
+  if (g_first >= n_groups) {
+    if (b.part) store_row<BLK>(b, nullptr);
+    return;
+  }
   const uint32_t copy = blockIdx.x & (b.n_copies - 1u);
   const bool do_model = (stages & STAGE_MODEL) != 0;
   const bool do_contrib = (stages & STAGE_CONTRIB) != 0;
@@ -1189,7 +1248,10 @@ __global__ void __launch_bounds__(BLK)
     }
   }
   __syncthreads();
-  flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
+  if (b.part)
+    store_row<BLK>(b, s_acc);
+  else
+    flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
 }
 
 // What the books read of a run, requested together (before its counter shards
@@ -1435,7 +1497,7 @@ __device__ __forceinline__ uint32_t request_prefix(const BatchDev& b, uint32_t s
 // records of the two steps are separate tables, the concentrations are
 // double-buffered), and the block that keeps the books also lays out the next
 // step's tiles, so the next step starts with its particle pass.  K: copies of
-// the accumulators (a variant each, as the copies' registers cost the others
+// the accumulators, or TAKE_ROWS (a variant each, as the copies' registers cost the others
 // occupancy: one copy's taking turns of 8 copies' code made the resolve kernel
 // of a 40-run batch 24 us instead of 20).
 template <class M, int K>
@@ -1476,7 +1538,10 @@ __global__ void __launch_bounds__(256, M::NV <= 8 ? 4 : 1) k_resolve(BatchDev b,
   uint32_t ev_run = 0, ev_moves = 0, ev_req = 0;  // movers and requests of the block's groups (thread 0)
   const bool leave_stage = (b.stages & STAGE_LEAVE) != 0;
   if (tr_block) {
-    transport_compartments<M, K>(b, runs, maps, blockIdx.x, tr_blocks, ahead);
+    if constexpr (K == TAKE_ROWS)
+      sum_rows<M>(b, runs, maps, blockIdx.x, tr_blocks, ahead);
+    else
+      transport_compartments<M, K>(b, runs, maps, blockIdx.x, tr_blocks, ahead);
   }
   for (uint32_t grp = rb; !tr_block && grp < n_groups; grp += n_res) {
     const uint32_t sc0 = grp * GS;
@@ -1939,18 +2004,25 @@ template <class M>
 void transport_t(const BatchDev& b, int grid, hipStream_t s) {
   hipLaunchKernelGGL(k_transport<M>, dim3(grid), dim3(256), 0, s, b, b.runs, b.maps);
 }
-template <class M>
-void resolve_t(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s) {
-  if (b.n_copies == 1)
-    hipLaunchKernelGGL((k_resolve<M, 1>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
-                       (const uint32_t*)b.tile_off, aux, ahead ? 1u : 0u);
-  else
-    hipLaunchKernelGGL((k_resolve<M, (int)run_copies(M::NS)>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
-                       (const uint32_t*)b.tile_off, aux, ahead ? 1u : 0u);
+template <class M, int K>
+static void launch_resolve(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s) {
+  hipLaunchKernelGGL((k_resolve<M, K>), dim3(grid + (int)aux), dim3(256), 0, s, b, b.runs, b.maps,
+                     (const uint32_t*)b.tile_off, aux, ahead ? 1u : 0u);
 }
 template <class M>
-const void* resolve_kernel_t(uint32_t copies) {
-  return copies == 1 ? (const void*)&k_resolve<M, 1> : (const void*)&k_resolve<M, (int)run_copies(M::NS)>;
+void resolve_t(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s) {
+  if (b.part)
+    launch_resolve<M, TAKE_ROWS>(b, grid, aux, ahead, s);
+  else if (b.n_copies == 1)
+    launch_resolve<M, 1>(b, grid, aux, ahead, s);
+  else
+    launch_resolve<M, (int)run_copies(M::NS)>(b, grid, aux, ahead, s);
+}
+template <class M>
+const void* resolve_kernel_t(const BatchDev& b) {
+  return b.part            ? (const void*)&k_resolve<M, TAKE_ROWS>
+         : b.n_copies == 1 ? (const void*)&k_resolve<M, 1>
+                           : (const void*)&k_resolve<M, (int)run_copies(M::NS)>;
 }
 template <class M>
 void properties_t(const BatchDev& b, uint32_t run, uint64_t n, uint32_t n_c, double* values, double* spatial,

@@ -15,7 +15,7 @@
 
 namespace mcst {
 
-constexpr uint32_t UDF_ABI_VERSION = 17;
+constexpr uint32_t UDF_ABI_VERSION = 18;
 
 struct UdfModel {
   uint32_t abi_version;
