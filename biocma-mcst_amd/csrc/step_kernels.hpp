@@ -2042,6 +2042,8 @@ void properties_t(const BatchDev& b, uint32_t run, uint64_t n, uint32_t n_c, dou
 // The launchers of model M's kernels.
 template <class M>
 ModelOps model_ops() {
+  static_assert(vars_declared_soundly<M>(),
+                "a model that declares READS declares WRITES too, and each has a bit per state variable at most");
   return ModelOps{&transport_t<M>, &launch_t<M>, &kernel_ptr_t<M>, &resolve_t<M>, &resolve_kernel_t<M>,
                   &properties_t<M>};
 }

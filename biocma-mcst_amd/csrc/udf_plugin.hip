@@ -10,7 +10,10 @@
 // mass); its ID member is not used: the library numbers loaded models itself.
 // record() writes exactly NR terms (r[0..NR); NR is NS unless the struct
 // declares it): the record row holds the move probability and the exit
-// threshold right after them.
+// threshold right after them.  A struct may declare which variables update()
+// reads and writes (READS and WRITES, a bit each; READS not without WRITES): the
+// others are then not loaded, not stored.  A variable written on some paths of
+// update() only must be in both.
 #include "step_kernels.hpp"
 #include "udf.hpp"
 
