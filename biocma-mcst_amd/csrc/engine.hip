@@ -751,9 +751,12 @@ int choose_launch(mcst_engine* e) {
   int best_waves = -1;
   for (int blk : order) {
     if (!priv && blk != 256) continue;
-    if (windowed && probe && blk == 1024) continue;
-    if (forced_block && blk != forced_block) continue;
-    const void* fn = M.ops->particle_kernel(blk, priv, false, priv && windowed, e->any_leave, small);
+    // a probing batch has its pass in 256 threads alone (with the exit tests
+    // always), whatever block is tuned or forced for the others (with the grid
+    // of one block of 512 per CU, half its waves, the pass of 3e6 particles in
+    // 3000 compartments took 58 us; with its own two per CU 45)
+    if (probe ? blk != 256 : forced_block && blk != forced_block) continue;
+    const void* fn = M.ops->particle_kernel(blk, priv, probe, priv && windowed, e->any_leave || probe, small);
     if (!fn) continue;
     const size_t lds = priv ? lds_need : 0;
     if (lds > 64 * 1024)
@@ -764,7 +767,7 @@ int choose_launch(mcst_engine* e) {
       continue;
     }
     hipFuncAttributes fa{};
-    if (hipFuncGetAttributes(&fa, fn) == hipSuccess && fa.localSizeBytes > 0 && !forced_block)
+    if (hipFuncGetAttributes(&fa, fn) == hipSuccess && fa.localSizeBytes > 0 && !forced_block && !probe)
       per_cu = per_cu / 2;  // register spills: prefer a variant that fits
     // waves per CU count up to 8, and a grid holds at most 8 waves per CU
     // (but one block of 1024); with a compartment window up to 16: its waves
@@ -790,16 +793,13 @@ int choose_launch(mcst_engine* e) {
     b.nsub = TILE / (64u * (uint32_t)M.nl);
     int per_cu = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, M.ops->particle_kernel(256, false, false, false, e->any_leave, false), 256, 0));
+        &per_cu, M.ops->particle_kernel(256, false, probe, false, e->any_leave || probe, false), 256, 0));
     best.grid = std::min(std::max(per_cu, 1), 2) * prop.multiProcessorCount;  // 8 waves per CU
   }
   const uint64_t groups = b.moved ? (uint64_t)b.T_max * b.nsub * 64 / best.block : b.T_max;  // at most
   best.grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)best.grid, groups));
   best.probe = probe;
   best.leave = e->any_leave;
-  if (best.probe && best.lds > 64 * 1024)
-    (void)hipFuncSetAttribute(M.ops->particle_kernel(256, best.priv, true, best.win, true, false),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)best.lds);
   // one run, or a window of compartments: blocks take groups in turn, which
   // keeps the wave front of the whole grid inside a narrow window of the
   // particle arrays (and, with a compartment window, centres it for each
@@ -2276,7 +2276,7 @@ int mcst_engine_autotune(mcst_engine* e, uint32_t steps, int32_t* block, int32_t
     e->tuned_block = blk;
     e->tuned_group = -1;
     if ((rc = choose_launch(e))) break;
-    if (e->plaunch.block != blk || (e->plaunch.probe && blk != 256)) continue;  // not resident / same kernel
+    if (e->plaunch.block != blk) continue;  // not resident, or a probing batch
     for (int g : {0, 1, 2, 4, 8}) {
       e->bd.tile_group = (uint32_t)g;
       double tot = 0.0, per[6] = {};
