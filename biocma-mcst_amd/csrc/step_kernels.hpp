@@ -749,10 +749,7 @@ __global__ void __launch_bounds__(BLK)
           acc_win = b.acc_w < acc_nc ? b.acc_w : acc_nc;
           if (tid == 0) {
             // wave 0 holds the group's first sub-chunk; its lane 0 the first slot
-            const uint32_t c0 = cur.cnt ? A.pos[0] : 0u;
-            const uint32_t half = acc_win / 2;
-            const uint32_t lo = c0 > half ? c0 - half : 0u;
-            s_w0 = lo + acc_win <= acc_nc ? lo : acc_nc - acc_win;
+            s_w0 = window_at(cur.cnt ? A.pos[0] : 0u, acc_win, acc_nc);
           }
           __syncthreads();
           acc_w0 = s_w0;
@@ -761,18 +758,15 @@ __global__ void __launch_bounds__(BLK)
         __syncthreads();
       } else if constexpr (WIN) {
         // the window follows the block's slots, looked at where a turn of the
-        // block begins (a block barrier per turn): when the turn's first
-        // compartment has left the window's middle half, flush it and centre
-        // it there
+        // block begins (a block barrier per turn): flushed where it moves
         if (acc_win < acc_nc && grp % G == 0) {
-          if (tid == 0) s_w0 = cur.cnt ? A.pos[0] : acc_w0 + acc_win / 2;
+          if (tid == 0) s_w0 = cur.cnt ? window_next(A.pos[0], acc_w0, acc_win, acc_nc) : acc_w0;
           __syncthreads();
-          const uint32_t c0 = s_w0;
+          const uint32_t w0 = s_w0;
           __syncthreads();  // every wave has read s_w0
-          if (c0 - (acc_w0 + acc_win / 4) >= acc_win / 2) {  // wraps when below
+          if (w0 != acc_w0) {
             flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
-            const uint32_t lo = c0 > acc_win / 2 ? c0 - acc_win / 2 : 0u;
-            acc_w0 = lo + acc_win <= acc_nc ? lo : acc_nc - acc_win;
+            acc_w0 = w0;
             __syncthreads();  // the flush has cleared every entry
           }
         }
