@@ -697,11 +697,13 @@ int choose_launch(mcst_engine* e) {
   HIP_TRY(hipGetDeviceProperties(&prop, e->device));
   size_t lds_need = 0;
   uint32_t live = 0;
+  uint64_t live_tiles = 0;
   bool probe = false;
   for (const auto& h : e->runs)
     if (h.phase == 1) {
       lds_need = std::max(lds_need, (size_t)h.n_s * h.n_c * sizeof(double));
       probe = probe || h.probe_cap > 0;
+      live_tiles += h.tiles;
       ++live;
     }
   const size_t lds_cap = std::min<size_t>(std::max(prop.sharedMemPerBlock, prop.sharedMemPerBlockOptin),
@@ -805,8 +807,16 @@ int choose_launch(mcst_engine* e) {
   // particle arrays (and, with a compartment window, centres it for each
   // group); a batch takes turns of 4 groups, so that a block changes runs less
   // often (40 uneven runs of 8.6e6 particles in all, 60 steps: 9164 us, turns
-  // of 2 and 8 10080 and 10180, one contiguous range per block 10090)
-  b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : (live <= 1 || windowed ? 1u : 4u);
+  // of 2 and 8 10080 and 10180, one contiguous range per block 10090).  In a
+  // batch with a compartment window a change of runs flushes a CU's whole LDS:
+  // where a block would meet a run per turn, as many runs as turns or more, it
+  // takes one range.  16 runs of 400 000 in 15 000 compartments, 2 species, a
+  // step in compartment order and mixed: one range 140 and 366 us, turns of one
+  // group 181 and 506; 8 of 50 000 to 1e6 in 6000, 4 species: 110 and 185, 106
+  // and 291; but 3 of 3e5 to 1.5e6 in 9000 to 30 000: 115 and 417, 100 and 434
+  const uint64_t turns = live_tiles * b.nsub * 64 / ((uint64_t)best.block * (uint64_t)best.grid);
+  const uint32_t group = live <= 1 ? 1u : !windowed ? 4u : turns > live ? 1u : 0u;
+  b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : group;
   if (const char* v = std::getenv("MCST_TILE_GROUP")) b.tile_group = (uint32_t)std::max(0, std::atoi(v));
   // copies of the accumulators: 8 for a batch of few enough values (each of its
   // runs then has 8 allocated), else one

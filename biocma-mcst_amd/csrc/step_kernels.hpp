@@ -757,9 +757,10 @@ __global__ void __launch_bounds__(BLK)
         for (uint32_t i = tid; i < acc_ns * acc_win; i += BLK) s_acc[i] = 0.0;
         __syncthreads();
       } else if constexpr (WIN) {
-        // the window follows the block's slots, looked at where a turn of the
-        // block begins (a block barrier per turn): flushed where it moves
-        if (acc_win < acc_nc && grp % G == 0) {
+        // the window follows the block's slots, looked at where a turn of one
+        // group begins, or every other group of a longer one (two block
+        // barriers each time): flushed where it moves
+        if (acc_win < acc_nc && (G == 1 || (grp & 1u) == 0)) {
           if (tid == 0) s_w0 = cur.cnt ? window_next(A.pos[0], acc_w0, acc_win, acc_nc) : acc_w0;
           __syncthreads();
           const uint32_t w0 = s_w0;
