@@ -401,7 +401,7 @@ struct HostRun {
   std::vector<uint32_t> vx_out;    // outlets whose first leaving feed is time-dependent ...
   std::vector<uint32_t> vx_feed;   // ... and that feed (index into vf)
   double* d_vf = nullptr;          // device: VF_ROWS rows of a step's flows of vf, then the outlets' thresholds
-  uint32_t vf_from = 0, vf_to = 0; // the steps those rows hold
+  uint32_t vf_from = 0, vf_to = 0; // the steps those rows hold (VF_ROWS at most)
   double ratio = 0.01;
   uint64_t min_removal = 0;
   uint32_t div_cap = 0xFFFFFFFFu; // newborns per step at most (the reference's division buffer)
@@ -1658,32 +1658,38 @@ void count_steps(mcst_engine* e, uint64_t k) {
 }
 
 // Flows of the time-dependent feeds for the step each live run is about to
-// take and the one after it, which that step's resolve kernel may transport (t
-// = step * dt, as update_feed), and the exit thresholds of the outlets they
-// lead, computed on the host like the constant feeds': VF_ROWS steps at a time.
-int prepare_feeds(mcst_engine* e) {
+// take and the one after it, if the call has one (`left` steps), which that
+// step's resolve kernel may transport (t = step * dt, as update_feed), and the
+// exit thresholds of the outlets they lead, computed on the host like the
+// constant feeds', for a block of steps (feed_rows).
+int prepare_feeds(mcst_engine* e, uint64_t left) {
   bool synced = false;
   std::vector<double> v;
   for (auto& h : e->runs) {
     if (h.phase != 1 || h.vf.empty() || h.host_step >= h.step_target) continue;
-    if (h.host_step >= h.vf_from && (uint64_t)h.host_step + 2 <= h.vf_to) continue;
+    const uint64_t need = std::min<uint64_t>(h.step_target, (uint64_t)h.host_step + (left > 1 ? 2 : 1));
+    if (h.host_step >= h.vf_from && need <= h.vf_to) continue;
     if (!synced) {  // the steps launched so far have read the rows they need
       HIP_TRY(hipStreamSynchronize(e->stream));
       synced = true;
     }
     const size_t w = h.vf.size() + h.vx_out.size();
-    v.assign(w * VF_ROWS, 0.0);
+    const uint32_t rows = feed_rows(h.host_step, h.step_target, left, h.vf_to - h.vf_from);
+    v.assign(w * rows, 0.0);
     h.vf_from = h.host_step;
-    h.vf_to = (uint32_t)std::min<uint64_t>((uint64_t)h.host_step + VF_ROWS, 0xFFFFFFFFull);
+    h.vf_to = h.host_step + rows;
     for (uint32_t step = h.vf_from; step < h.vf_to; ++step) {
-      double* row = v.data() + (size_t)(step % VF_ROWS) * w;
+      double* row = v.data() + (size_t)(step - h.vf_from) * w;
       const double t = (double)step * h.dt;
       for (size_t q = 0; q < h.vf.size(); ++q) row[q] = feed_flow(h.feeds[h.vf[q]], t);
       const HostMap& mp = h.maps[(step / h.steps_per_map) % h.maps.size()];
       for (size_t x = 0; x < h.vx_out.size(); ++x)
         row[h.vf.size() + x] = std::exp(-(h.dt * row[h.vx_feed[x]]) / mp.V[h.vx_out[x]]);
     }
-    HIP_TRY(hipMemcpy(h.d_vf, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice));
+    const uint32_t at = h.vf_from % VF_ROWS, head = std::min(rows, VF_ROWS - at);  // then from row 0 on
+    HIP_TRY(hipMemcpy(h.d_vf + at * w, v.data(), head * w * sizeof(double), hipMemcpyHostToDevice));
+    if (rows > head)
+      HIP_TRY(hipMemcpy(h.d_vf, v.data() + head * w, (rows - head) * w * sizeof(double), hipMemcpyHostToDevice));
   }
   return MCST_OK;
 }
@@ -1698,13 +1704,13 @@ bool can_transport_ahead(const mcst_engine* e, uint32_t stages) {
   return stages == STAGE_ALL && !has_growth(e);
 }
 
-// One step of the batch, then the reorders that fall due (transported,
-// ahead: as launch_step).
-int step_once(mcst_engine* e, uint32_t stages, const hipEvent_t* ev = nullptr, bool transported = false,
+// One step of the batch, the first of `left` of the call, then the reorders
+// that fall due (transported, ahead: as launch_step).
+int step_once(mcst_engine* e, uint32_t stages, uint64_t left, const hipEvent_t* ev = nullptr, bool transported = false,
               bool ahead = false) {
   const int rcg = grow_runs(e);
   if (rcg) return rcg;
-  const int rcf = prepare_feeds(e);
+  const int rcf = prepare_feeds(e, left);
   if (rcf) return rcf;
   std::vector<uint32_t> before(e->runs.size());
   for (size_t r = 0; r < e->runs.size(); ++r) before[r] = e->runs[r].host_step;
@@ -2211,7 +2217,7 @@ int mcst_engine_step(mcst_engine* e, uint32_t n_steps) {
   // reads between calls is the same either way
   const bool ahead = can_transport_ahead(e, STAGE_ALL);
   for (uint32_t k = 0; k < n_steps; ++k) {
-    const int rc = step_once(e, STAGE_ALL, nullptr, ahead && k > 0, ahead && k + 1 < n_steps);
+    const int rc = step_once(e, STAGE_ALL, n_steps - k, nullptr, ahead && k > 0, ahead && k + 1 < n_steps);
     if (rc) return rc;
   }
   HIP_TRY(hipGetLastError());
@@ -2223,7 +2229,7 @@ int mcst_engine_step_stages(mcst_engine* e, uint32_t stages) {
   if (!e->committed) return fail(MCST_ERR_STATE, "engine not committed");
   if (stages & ~STAGE_ALL) return fail(MCST_ERR_ARG, "unknown stage bits");
   HIP_TRY(hipSetDevice(e->device));
-  const int rc = step_once(e, stages);
+  const int rc = step_once(e, stages, 1);
   if (rc) return rc;
   HIP_TRY(hipGetLastError());
   return MCST_OK;
@@ -2346,7 +2352,7 @@ int mcst_engine_profile(mcst_engine* e, uint32_t n_steps, double* total_ms, doub
   // flows, reorders), with events between the kernels
   const uint32_t steps = e->bd.R ? n_steps : 0;
   for (uint32_t s = 0; s < steps; ++s) {
-    const int rc = step_once(e, STAGE_ALL, &ev[(size_t)s * (K + 1)]);
+    const int rc = step_once(e, STAGE_ALL, steps - s, &ev[(size_t)s * (K + 1)]);
     if (rc) return rc;
   }
   HIP_TRY(hipEventRecord(t1, e->stream));

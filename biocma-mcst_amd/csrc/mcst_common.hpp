@@ -113,12 +113,21 @@ struct MapDev {
 };
 constexpr uint32_t MOVE_ROW_M = 6;
 
-// Steps of time-dependent feeds the host prepares at once: their flows depend
-// on the step number alone.  (Prepared before every step, they cost a wait for
+// Steps of time-dependent feeds the host prepares at once at most: their flows
+// depend on the step number alone.  (Prepared before every step, they cost a wait for
 // the stream and a copy each time, and kept the next step's transport out of
 // the resolve kernel: 20 011 particles of a two-phase column 50 us a step, now
 // 25.)
 constexpr uint32_t VF_ROWS = 256;
+// Rows to prepare from `step` on, for a call with `left` steps to take: those
+// steps, or twice the rows of the last time, so that single steps are prepared
+// in ever longer blocks and nobody pays for more than twice what they use (a row
+// of many outlets is as many exponentials); none past the run's last step.
+constexpr uint32_t feed_rows(uint32_t step, uint32_t target, uint64_t left, uint32_t last) {
+  const uint64_t want = left > 2ull * last ? left : 2ull * last;
+  const uint64_t most = target - step < VF_ROWS ? target - step : VF_ROWS;
+  return (uint32_t)(want < most ? want : most);
+}
 
 // vf_src_s / vf_sink_k entries that belong to the gas phase
 constexpr uint32_t VF_GAS = 0x80000000u;
