@@ -46,7 +46,10 @@ class Result:
 def footprint(case, n_var):
     """Device bytes a run holds while resident: its slot range (state, the
     two base ages and their clock origins, position, status and the pass's
-    mover and division lists), its flowmaps and liquid arrays."""
+    mover and division lists), its flowmaps, its liquid arrays (among them the
+    copies of its contributions: run_copies and S_COPY_ENTRIES of the library)
+    and the rows of its time-dependent feeds (VF_ROWS steps of each feed's flow
+    and of the exit threshold of each outlet that one leads)."""
     cap = case.capacity or 2 * case.n_particles
     slots = -(-cap // TILE) * TILE
     per_slot = 8 * n_var + 2 * 8 + 2 * 4 + 4 + 1 + 3 * 4
@@ -55,8 +58,18 @@ def footprint(case, n_var):
         deg = max(1, int(max(1, (len(flows) + case.n_c - 1) // case.n_c)))
         maps += case.n_c * (8 * 4 + 12 * 2 * deg) + 20 * (len(flows) + case.n_c)
     entries = case.n_s * case.n_c
-    liquid = 8 * (6 + ((8 if case.n_s <= 2 else 2) if entries <= 16384 else 1)) * entries
-    return slots * per_slot + maps + liquid
+    copies = {1: 8, 2: 4}.get(case.n_s, 2) if entries <= 16384 else 1
+    liquid = 8 * (6 + copies) * entries
+    feeds = getattr(case, "feeds", None) or []
+    gas = (getattr(case, "two_phase", None) or {}).get("gas_feeds", [])
+    leads = {}  # outlet -> kind of the first feed that leaves there
+    for kind, _, _, _, out, *_ in feeds:
+        if out is not None and out >= 0:
+            leads.setdefault(out, kind)
+    kinds = [f[0] for f in feeds] + [f[0] for f in gas]
+    timed = sum(k != "constant" for k in kinds)
+    rows = 256 * 8 * (timed + sum(k != "constant" for k in leads.values())) if timed else 0
+    return slots * per_slot + maps + liquid + rows
 
 
 class Server:
