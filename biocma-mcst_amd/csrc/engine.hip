@@ -815,7 +815,9 @@ int choose_launch(mcst_engine* e) {
   // group 181 and 506; 8 of 50 000 to 1e6 in 6000, 4 species: 110 and 185, 106
   // and 291; but 3 of 3e5 to 1.5e6 in 9000 to 30 000: 115 and 417, 100 and 434
   const uint64_t turns = live_tiles * b.nsub * 64 / ((uint64_t)best.block * (uint64_t)best.grid);
-  const uint32_t group = live <= 1 ? 1u : !windowed ? 4u : turns > live ? 1u : 0u;
+  // (the small pass: one group at a time, in a batch one range per block, which
+  // meets few runs)
+  const uint32_t group = b.moved ? (b.R == 1 ? 1u : 0u) : live <= 1 ? 1u : !windowed ? 4u : turns > live ? 1u : 0u;
   b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : group;
   if (const char* v = std::getenv("MCST_TILE_GROUP")) b.tile_group = (uint32_t)std::max(0, std::atoi(v));
   // copies of the accumulators: 8 for a batch of few enough values (each of its

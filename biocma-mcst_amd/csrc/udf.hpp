@@ -15,7 +15,7 @@
 
 namespace mcst {
 
-constexpr uint32_t UDF_ABI_VERSION = 18;
+constexpr uint32_t UDF_ABI_VERSION = 19;
 
 struct UdfModel {
   uint32_t abi_version;
