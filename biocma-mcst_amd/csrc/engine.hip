@@ -815,11 +815,13 @@ int choose_launch(mcst_engine* e) {
   // group 181 and 506; 8 of 50 000 to 1e6 in 6000, 4 species: 110 and 185, 106
   // and 291; but 3 of 3e5 to 1.5e6 in 9000 to 30 000: 115 and 417, 100 and 434
   const uint64_t turns = live_tiles * b.nsub * 64 / ((uint64_t)best.block * (uint64_t)best.grid);
-  // (the small pass: one group at a time, in a batch one range per block, which
-  // meets few runs)
+  // (the small pass knows turns of one group and one range per block, which
+  // meets few runs of a batch: with turns of any length the scalars of its loop
+  // spill, 0.2 us of a pass of 5)
   const uint32_t group = b.moved ? (b.R == 1 ? 1u : 0u) : live <= 1 ? 1u : !windowed ? 4u : turns > live ? 1u : 0u;
   b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : group;
   if (const char* v = std::getenv("MCST_TILE_GROUP")) b.tile_group = (uint32_t)std::max(0, std::atoi(v));
+  if (b.moved && b.tile_group != 1u) b.tile_group = 0u;
   // copies of the accumulators: 8 for a batch of few enough values (each of its
   // runs then has 8 allocated), else one
   uint64_t entries = 0;
@@ -2296,6 +2298,7 @@ int mcst_engine_autotune(mcst_engine* e, uint32_t steps, int32_t* block, int32_t
     if ((rc = choose_launch(e))) break;
     if (e->plaunch.block != blk) continue;  // not resident, or a probing batch
     for (int g : {0, 1, 2, 4, 8}) {
+      if (e->bd.moved && g > 1) break;  // the small pool's pass knows these two
       e->bd.tile_group = (uint32_t)g;
       double tot = 0.0, per[6] = {};
       if ((rc = mcst_engine_profile(e, steps, &tot, per))) break;

@@ -1095,10 +1095,12 @@ __global__ void __launch_bounds__(BLK)
   const uint64_t P = b.P;
   const uint32_t n_sc = tile_off[R] * NSUB;
   const uint32_t n_groups = (n_sc + WPB - 1) / WPB;
-  // groups dealt to the blocks in turns, as in k_particle
+  // groups dealt to the blocks one at a time, or one range per block
   const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
-  const uint32_t G = b.tile_group && b.tile_group < chunk ? b.tile_group : chunk;
-  if (blockIdx.x * G >= n_groups) {  // the whole block; or no groups at all
+  const bool deal = b.tile_group == 1u;
+  const uint32_t g_first = deal ? blockIdx.x : blockIdx.x * chunk, g_step = deal ? gridDim.x : 1u;
+  const uint32_t g_end = deal || n_groups - g_first < chunk ? n_groups : g_first + chunk;
+  if (g_first >= n_groups) {
     if (b.part) store_row<BLK>(b, nullptr);
     return;
   }
@@ -1107,9 +1109,7 @@ __global__ void __launch_bounds__(BLK)
   const bool do_contrib = (stages & STAGE_CONTRIB) != 0;
   uint32_t acc_run = 0xFFFFFFFFu, acc_ns = 0, acc_nc = 0;
   GLOBAL_AS double* acc_S = nullptr;
-  uint32_t turn = blockIdx.x * G;
-  for (uint32_t grp = turn, g_next; grp < n_groups; grp = g_next) {
-    g_next = grp + 1u < turn + G ? grp + 1u : (turn += gridDim.x * G);
+  for (uint32_t grp = g_first; grp < g_end; grp += g_step) {
     // ---- the wave's sub-chunk; none past the last (every wave meets the
     // block's barriers)
     const uint32_t sc = grp * WPB + wave;
