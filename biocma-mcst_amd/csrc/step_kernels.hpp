@@ -1217,8 +1217,15 @@ __global__ void __launch_bounds__(BLK)
         gp(b.div_rec)[seg + rk] = (slot % TILE) | (pv << LIST_POS_SHIFT);
         gp(b.div_pos)[seg + rk] = pos;
       }
-      // (a small pool's one entry of 2^18 sub-chunks is never read)
-      if (lane < 2) atomicAdd((lane ? b.div_l2 : b.div_l1) + (sc >> (lane ? 12 : 6)), n_div);
+      // of the block counts, those of 64 sub-chunks alone (request_prefix): with
+      // an atomic per sub-chunk on a count of 4096 as well, 8e5 cells in a full
+      // container, a quarter of them asking in every step, had a pass of 106 us,
+      // nearly all of it those atomics one after another; now 49
+      // (the index in a vector register: for an address that it knows to be the
+      // wave's the compiler puts a reduction over the wave before the atomic)
+      uint32_t i1 = sc >> 6;
+      asm volatile("" : "+v"(i1));
+      if (lane == 0) atomicAdd(b.div_l1 + i1, n_div);
     }
     // ---- stores
     if (idle && do_model) {
@@ -1473,15 +1480,17 @@ static_assert(RES_SC <= 256 && 32 % NSUB_MAX == 0, "a group is at most one sub-c
 
 // Requests of the pass in sub-chunks [0, sc), summed by one wave from the
 // block counts (div_l3, div_l2, div_l1: blocks of 2^18, 2^12 and 2^6
-// sub-chunks) and the sub-chunk counts of sc's own block of 64.
+// sub-chunks; in a small pool div_l1 alone, 768 at most) and the sub-chunk
+// counts of sc's own block of 64.
 __device__ __forceinline__ uint32_t request_prefix(const BatchDev& b, uint32_t sc, uint32_t lane) {
   const uint32_t a3 = sc >> 18, a2 = sc >> 12, a1 = sc >> 6;
   uint32_t v = 0;
   for (uint32_t i = lane; i < a3; i += 64) v += b.div_l3[i];
-  const uint32_t i2 = (a3 << 6) + lane, i1 = (a2 << 6) + lane, i0 = (a1 << 6) + lane;
+  const uint32_t i2 = (a3 << 6) + lane, i1 = (b.moved ? 0u : a2 << 6) + lane, i0 = (a1 << 6) + lane;
   const uint32_t x2 = i2 < a2 ? b.div_l2[i2] : 0u;
-  const uint32_t x1 = i1 < a1 ? b.div_l1[i1] : 0u;
   const uint32_t x0 = i0 < sc ? b.sub_divs[i0] : 0u;
+  uint32_t x1 = 0;  // one round but in a small pool
+  for (uint32_t i = i1; i < a1; i += 64) x1 += b.div_l1[i];
   return wave_sum(v + x2 + x1 + x0);
 }
 
