@@ -48,13 +48,15 @@ constexpr uint32_t LIST_POS_SHIFT = 11;
 constexpr uint32_t LIST_POS_FAR = 0xFFFFFFFFu >> LIST_POS_SHIFT;
 static_assert(TILE <= MOVER_INACTIVE, "a tile-local slot fits below the flag");
 
-// Largest pool, in tiles, that the small batch's particle pass serves.  Measured
-// per step against the pipelined pass: 100 000 particles of 2 states 15.0 us
-// against 19.6, 345 679 of 3 23.5 and 25.4, 250 003 of 8 (2 slots per lane) 40.2
-// and 40.5, and level at 1e6 (27-50 us).  Where the pipelined pass holds many
-// states of 4 slots per lane its registers leave it few waves and the line lies
-// further up: 1e6 of 6 states 37.3 and 41.8 us, 1e6 of 9 58.5 and 72.9, 3e6 of 9
-// 181 and 157.
+// Largest pool, in tiles, that the small batch's particle pass serves.  A step
+// with the pipelined pass and with this one: 500 000 particles of 2, 3 and 8
+// states (the last with 2 slots per lane) 25, 22.6, 32.9 us and 24, 22.2, 30.3;
+// 1e6 29.4, 28.1, 42.0 and 30.6, 28.0, 41.0: the line.  Where the pipelined pass
+// holds many states of 4 slots per lane its registers leave it few waves and the
+// line lies further up: 6 states 1e6 34.5 and 34.7, 2e6 51.0 and 47.4, 3e6 64.2
+// and 59.7, 5e6 91.9 and 91.9; 9 states 1e6 50.6 and 47.0, 2e6 77.6 and 70-80,
+// 3e6 107 and 138, which a pool of these tiles holds only when it is full (its
+// slots are what is known here, and a run has twice its particles by default).
 constexpr uint32_t small_tiles(int nv, int nl) { return nv * nl >= 24 ? 3072u : 1024u; }
 
 // Stage mask of one step (values shared with the C ABI).
