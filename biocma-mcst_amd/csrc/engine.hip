@@ -774,8 +774,9 @@ int choose_launch(mcst_engine* e) {
     // waves per CU count up to 8, and a grid holds at most 8 waves per CU
     // (but one block of 1024); with a compartment window up to 16: its waves
     // also wait on window flushes and the global atomics of the particles
-    // outside it.  Twice the waves: 1e7 particles 3245 us for 20 steps against
-    // 3198, 3e6 particles 2919 against 2922 for 40
+    // outside it.  Twice the waves, measured with the loads and stores of today's
+    // models: 1e7 particles 2957 us for 20 steps against 2919, 3e6 particles 2893
+    // against 2830 for 40 (a batch of 40 uneven runs 8160 against 8830 for 60)
     const int wcap = windowed || small ? 16 : 8;
     const int use = std::min(per_cu, std::max(1, wcap * 64 / blk));
     const int waves = std::min(use * blk / 64, wcap);
@@ -806,8 +807,8 @@ int choose_launch(mcst_engine* e) {
   // keeps the wave front of the whole grid inside a narrow window of the
   // particle arrays (and, with a compartment window, centres it for each
   // group); a batch takes turns of 4 groups, so that a block changes runs less
-  // often (40 uneven runs of 8.6e6 particles in all, 60 steps: 9164 us, turns
-  // of 2 and 8 10080 and 10180, one contiguous range per block 10090).  In a
+  // often (40 uneven runs of 8.6e6 particles in all, 60 steps: 8720 us, turns
+  // of 2 and 8 9390 and 9430, one contiguous range per block 8870).  In a
   // batch with a compartment window a change of runs flushes a CU's whole LDS:
   // where a block would meet a run per turn, as many runs as turns or more, it
   // takes one range.  16 runs of 400 000 in 15 000 compartments, 2 species, a
@@ -822,8 +823,8 @@ int choose_launch(mcst_engine* e) {
   b.tile_group = e->tuned_group >= 0 ? (uint32_t)e->tuned_group : group;
   if (const char* v = std::getenv("MCST_TILE_GROUP")) b.tile_group = (uint32_t)std::max(0, std::atoi(v));
   if (b.moved && b.tile_group != 1u) b.tile_group = 0u;
-  // copies of the accumulators: 8 for a batch of few enough values (each of its
-  // runs then has 8 allocated), else one
+  // copies of the accumulators: 8, 4 or 2 for a batch of few enough values (each
+  // of its runs then has as many allocated), else one
   uint64_t entries = 0;
   for (const auto& h : e->runs)
     if (h.phase == 1) entries += (uint64_t)h.n_s * h.n_c;
@@ -866,7 +867,7 @@ int choose_launch(mcst_engine* e) {
   e->grid_transport = (int)std::min<uint64_t>(((uint64_t)b.n_chunk_total + 3) / 4, 8192) + 1;
   // resolve: enough blocks for groups of 32 sub-chunks, up to the blocks
   // that are resident at once (a second round of blocks would start after
-  // the first had worked through their groups); the kernel picks 32 or 64
+  // the first had worked through their groups); the kernel picks 32 or 64 (128 of 64 slots)
   // from the step's tile count
   int res_per_cu = 0;
   HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&res_per_cu, M.ops->resolve_kernel(b), 256, 0));

@@ -164,7 +164,7 @@ constexpr int record_terms() {
 // cells that divide.
 template <class M>
 constexpr uint32_t all_vars() {
-  return M::NV >= 32 ? 0xFFFFFFFFu : (1u << M::NV) - 1u;
+  return (1u << M::NV) - 1u;  // at most MAX_VAR
 }
 template <class M, class = void>
 struct VarsRead {
@@ -182,14 +182,13 @@ template <class M>
 struct VarsWritten<M, decltype((void)M::WRITES)> {
   static constexpr uint32_t value = M::WRITES;
 };
-// (variables past the 32nd count as read and written)
 template <class M>
 constexpr bool reads_var(int v) {
-  return v >= 32 || ((VarsRead<M>::value >> v) & 1u);
+  return (VarsRead<M>::value >> v) & 1u;
 }
 template <class M>
 constexpr bool writes_var(int v) {
-  return v >= 32 || ((VarsWritten<M>::value >> v) & 1u);
+  return (VarsWritten<M>::value >> v) & 1u;
 }
 
 template <class M, class = void>

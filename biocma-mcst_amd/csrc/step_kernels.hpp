@@ -80,7 +80,6 @@ __device__ __forceinline__ uint32_t find_run(const uint32_t* off, uint32_t R, ui
 }
 
 constexpr uint32_t SCAN_THREADS = 1024;
-constexpr uint32_t SCAN_WAVES = SCAN_THREADS / 64;
 
 }  // namespace
 
@@ -167,9 +166,10 @@ struct ColumnInflow {
 // whenever the host can read it.  TAKE_ROWS: the contributions are `given`,
 // summed from the rows by the caller.
 //
-// Every load comes before the first store (the arrays may alias as far as the
-// compiler knows: a store in between made it read the run's and the flowmap's
-// fields again, a round trip each).
+// Every load of a run without a gas phase comes before the first store (the
+// arrays may alias as far as the compiler knows: a store in between made it read
+// the run's and the flowmap's fields again, a round trip each); with one, the
+// gas is stored first, which spares its registers to the liquid's inflow.
 constexpr int TAKE_ROWS = -1;
 template <class M, int TAKE>
 __device__ __forceinline__ void transport_one(const BatchDev& b, const RunDev* __restrict__ runs,
@@ -1456,8 +1456,8 @@ __device__ void bookkeep_pass(const BatchDev& b, const RunDev* __restrict__ runs
   for (uint32_t i = tid; i <= RESOLVE_TICKETS; i += NT) b.ticket[i * TICKET_STRIDE] = 0u;
 }
 
-// After the particle pass, per group of 32 or 64 sub-chunks (one per thread
-// of the block for the prefix sums): (1) the movers the pass listed take
+// After the particle pass, per group of 32 or 64 sub-chunks, 128 after the small
+// pool's pass (one per thread of the block for the prefix sums): (1) the movers the pass listed take
 // their neighbour, the first CDF column at or above u, and an Idle one runs
 // the exit test in its new compartment (move_kernel.hpp:392-437, 586-648);
 // (2) the division requests are accepted in slot order over the whole run:
@@ -1915,7 +1915,7 @@ static void launch_particle_t(const BatchDev& b, int grid, size_t lds, hipStream
 }
 
 // The variants: direct global atomics (256 threads); an LDS accumulator of
-// whole runs (256/512/1024) or of a compartment window (256/512); each with
+// whole runs or of a compartment window (256/512/1024 both); each with
 // and without the leaving-flow work; and the 256-thread probe variants of
 // each accumulator kind (with it).
 template <class M, bool LV>
