@@ -401,6 +401,7 @@ struct HostRun {
   std::vector<uint32_t> vx_out;    // outlets whose first leaving feed is time-dependent ...
   std::vector<uint32_t> vx_feed;   // ... and that feed (index into vf)
   double* d_vf = nullptr;          // device: VF_ROWS rows of a step's flows of vf, then the outlets' thresholds
+  double* d_sp = nullptr;          // device: the run's own copies of its contribution accumulator (RunDev::Sp)
   uint32_t vf_from = 0, vf_to = 0; // the steps those rows hold (VF_ROWS at most)
   double ratio = 0.01;
   uint64_t min_removal = 0;
@@ -478,7 +479,7 @@ struct mcst_engine {
   uint32_t* alt_clk_div = nullptr;
   uint64_t alt_P = 0;
   uint32_t layout = 0;              // which of the two tile tables the step under way reads (launch_step)
-  double* part_mem = nullptr;       // contribution rows of the particle pass (BatchDev::part), part_bytes allocated
+  double* part_mem = nullptr;       // contribution rows of the particle pass (BatchDev::rows), part_bytes allocated
   size_t part_bytes = 0;
   int grid_aux = 1;                 // the resolve kernel's blocks that take the contributions
   int tuned_group = -1;
@@ -830,17 +831,19 @@ int choose_launch(mcst_engine* e) {
     if (h.phase == 1) entries += (uint64_t)h.n_s * h.n_c;
   b.n_copies = entries <= S_COPY_ENTRIES ? run_copies(M.ns) : 1u;
   // contribution rows (MCST_CONTRIB_ROWS=1; one live run whose whole
-  // accumulator is in LDS): each block of the pass stores its accumulator as
-  // a row and the resolve kernel sums the rows in a fixed order, instead of
-  // each block adding its accumulator to a copy with FP64 atomics.  Pass and
-  // resolve kernel of 1e7 particles in 5000 compartments (512 rows) 115 and
-  // 21.8 us against 116 and 20.1, of 1e5 in 64 (391 rows) 4.8 and 16.0 against
-  // 5.0 and 6.6: the atomics stay the default.
-  b.part = nullptr;
-  b.part_rows = b.part_w = 0;
+  // accumulator is in LDS): a copy for every block of the pass, summed by the
+  // resolve kernel in a fixed order.  Pass and resolve kernel of 1e7 particles in
+  // 5000 compartments (512 rows) 117 and 24.4 us against 116 and 20.1, of 1e5 in 64
+  // (391 rows) 4.8 and 19.9 against 4.6 and 7.0: the few copies stay the default.
+  // (Rows stored whole by the pass, without atomics, took 115 and 21.8, but their
+  // code cost the pass of a batch, which has none, 2 %.)
+  b.rows = 0;
   const char* rows = std::getenv("MCST_CONTRIB_ROWS");
+  uint32_t row_run = 0xFFFFFFFFu;
   if (rows && std::atoi(rows) != 0 && live == 1 && best.priv && !best.win) {
-    const size_t bytes = (size_t)best.grid * entries * sizeof(double);
+    uint32_t copies = 1;
+    while (copies < (uint32_t)best.grid) copies *= 2;
+    const size_t bytes = (size_t)copies * entries * sizeof(double);
     if (bytes > e->part_bytes) {  // a larger row buffer
       HIP_TRY(hipStreamSynchronize(e->stream));
       drop_graph(e);
@@ -851,15 +854,23 @@ int choose_launch(mcst_engine* e) {
         e->part_bytes = 0;
       }
       if (dev_alloc(e, (void**)&e->part_mem, bytes) == MCST_OK) e->part_bytes = bytes;
+      if (e->part_mem) HIP_TRY(hipMemset(e->part_mem, 0, bytes));  // the resolve kernel leaves it so
     }
     if (e->part_mem && bytes <= e->part_bytes) {
-      b.part = e->part_mem;
-      b.part_rows = (uint32_t)best.grid;
-      b.part_w = (uint32_t)entries;
-      b.n_copies = 1;
+      b.rows = (uint32_t)best.grid;
+      b.n_copies = copies;
+      for (uint32_t r = 0; r < e->runs.size(); ++r)
+        if (e->runs[r].phase == 1) row_run = r;
     }
   }
-  const uint32_t chunks_per_block = b.part ? 1 : 4;
+  for (uint32_t r = 0; r < e->runs.size(); ++r) {  // where each run's pass adds its contributions
+    if (e->runs[r].phase != 1) continue;
+    double* const sp = r == row_run ? e->part_mem : e->runs[r].d_sp;
+    if (e->h_runs[r].Sp == sp) continue;
+    e->h_runs[r].Sp = sp;
+    HIP_TRY(hipMemcpy(e->d_runs + r, &e->h_runs[r], sizeof(RunDev), hipMemcpyHostToDevice));
+  }
+  const uint32_t chunks_per_block = b.rows ? 1 : 4;
   e->grid_aux = (int)std::min<uint64_t>(((uint64_t)b.n_chunk_total + chunks_per_block - 1) / chunks_per_block, 8192);
   e->plaunch = best;
   e->grid_particle = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)prop.multiProcessorCount * 4, b.T_max));
@@ -877,7 +888,7 @@ int choose_launch(mcst_engine* e) {
   if (std::getenv("MCST_VERBOSE"))
     std::fprintf(stderr, "[mcst] particle pass: block=%d grid=%d lds=%zu priv=%d group=%u window=%u leave=%d copies=%u rows=%u (lds cap %zu)\n",
                  best.block, best.grid, best.lds, (int)best.priv, b.tile_group, b.acc_w, (int)best.leave,
-                 b.n_copies, b.part_rows, lds_cap);
+                 b.n_copies, b.rows, lds_cap);
   return MCST_OK;
 }
 
@@ -992,6 +1003,7 @@ int upload_run(mcst_engine* e, uint32_t r) {
   if ((rc = run_upload(h, &d.S, h.restored ? h.r_S.data() : zeros.data(), nsc))) return rc;
   const size_t n_sp = nsc * (nsc <= S_COPY_ENTRIES ? run_copies(e->model->ns) : 1u);
   if ((rc = run_alloc(h, (void**)&d.Sp, n_sp * sizeof(double)))) return rc;
+  h.d_sp = d.Sp;
   HIP_TRY(hipMemset(d.Sp, 0, n_sp * sizeof(double)));
   if ((rc = run_upload(h, (double**)&d.F, F.data(), nsc))) return rc;
   if ((rc = run_upload(h, (double**)&d.sink, sink.data(), sink.size()))) return rc;

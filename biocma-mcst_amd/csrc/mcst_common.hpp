@@ -295,12 +295,10 @@ struct BatchDev {
   // sums the copies
   uint32_t n_copies;
   // contribution rows (one live run whose whole [n_s][n_c] accumulator fits
-  // LDS): block k of the particle pass stores its accumulator at
-  // part[k * part_w], part_w = n_s * n_c, and the resolve kernel sums the
-  // part_rows rows in a fixed order; null: the copies above
-  double* part;
-  uint32_t part_rows;
-  uint32_t part_w;
+  // LDS): a copy for every block of the particle pass (n_copies is a power of two
+  // past them), so that each holds one block's sums, and the resolve kernel adds
+  // these `rows` copies in a fixed order; 0: the copies above
+  uint32_t rows;
   // the next step's tile_off, written by the books while blocks of the step may yet read tile_off
   uint32_t* tile_off_next;
 };

@@ -344,8 +344,8 @@ __device__ void transport_compartments(const BatchDev& b, const RunDev* __restri
 }
 
 // With contribution rows: as transport_compartments, a block taking 64
-// compartments.  Each of its waves sums a quarter of the rows, 8 in flight, and the
-// first adds the waves' sums in turn: the order is the rows' alone.
+// compartments.  Each of its waves sums (and clears) a quarter of the rows, 8 in
+// flight, and the first adds the waves' sums in turn: the order is the rows' alone.
 template <class M>
 __device__ void sum_rows(const BatchDev& b, const RunDev* __restrict__ runs, const MapDev* __restrict__ maps,
                          uint32_t blk, uint32_t n_blk, uint32_t ahead) {
@@ -361,11 +361,23 @@ __device__ void sum_rows(const BatchDev& b, const RunDev* __restrict__ runs, con
 #pragma unroll
     for (int s = 0; s < NS; ++s) t[s] = 0.0;
     if (j < n_c) {
-      const GLOBAL_AS double* const part = gp(b.part) + j;
-#pragma unroll 8
-      for (uint32_t row = wave; row < b.part_rows; row += NWV)
+      GLOBAL_AS double* const part = gp(runs[r].Sp) + j;
+      constexpr uint32_t RG = 8;
+      for (uint32_t row = wave; row < b.rows; row += RG * NWV) {
+        double x[RG][NS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) t[s] += part[(size_t)row * b.part_w + (size_t)s * n_c];
+        for (uint32_t k = 0; k < RG; ++k)
+#pragma unroll
+          for (int s = 0; s < NS; ++s)
+            x[k][s] = row + k * NWV < b.rows ? part[((size_t)(row + k * NWV) * NS + s) * n_c] : 0.0;
+#pragma unroll
+        for (uint32_t k = 0; k < RG; ++k)
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            t[s] += x[k][s];
+            if (row + k * NWV < b.rows) part[((size_t)(row + k * NWV) * NS + s) * n_c] = 0.0;
+          }
+      }
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) s_sum[wave][s][lane] = t[s];
@@ -427,14 +439,6 @@ __device__ __forceinline__ void flush_window(double* s_acc, GLOBAL_AS double* S,
       s_acc[i] = 0.0;
     }
   }
-}
-
-// With contribution rows: the block's row, from its LDS accumulator (null: of
-// a block without slots).
-template <int BLK>
-__device__ __forceinline__ void store_row(const BatchDev& b, const double* s_acc) {
-  GLOBAL_AS double* const row = gp(b.part) + (size_t)blockIdx.x * b.part_w;
-  for (uint32_t i = threadIdx.x; i < b.part_w; i += BLK) row[i] = s_acc ? s_acc[i] : 0.0;
 }
 
 // First column of a cumulative row with cp[c] >= u, clamped to m-1: for a
@@ -598,10 +602,7 @@ __global__ void __launch_bounds__(BLK)
   const uint32_t chunk = (n_groups + gridDim.x - 1) / gridDim.x;
   const uint32_t G = b.tile_group && b.tile_group < chunk ? b.tile_group : (chunk ? chunk : 1u);
   uint32_t grp = blockIdx.x * G;
-  if (grp >= n_groups) {  // the whole block
-    if (PRIV && !WIN && b.part) store_row<BLK>(b, nullptr);
-    return;
-  }
+  if (grp >= n_groups) return;  // the whole block
   const uint32_t copy = blockIdx.x & (b.n_copies - 1u);  // of each run's accumulator
   auto next_group = [&](uint32_t g) -> uint32_t {
     const uint32_t g0 = g - g % G;
@@ -1061,10 +1062,7 @@ __global__ void __launch_bounds__(BLK)
   }
   if (PRIV) {
     __syncthreads();
-    if (!WIN && b.part)
-      store_row<BLK>(b, s_acc);
-    else
-      flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
+    flush_window<BLK>(s_acc, acc_S, acc_ns, acc_win, acc_nc, acc_w0, tid);
   }
   flush_counts();
 #pragma unroll
@@ -1100,10 +1098,7 @@ __global__ void __launch_bounds__(BLK)
   const bool deal = b.tile_group == 1u;
   const uint32_t g_first = deal ? blockIdx.x : blockIdx.x * chunk, g_step = deal ? gridDim.x : 1u;
   const uint32_t g_end = deal || n_groups - g_first < chunk ? n_groups : g_first + chunk;
-  if (g_first >= n_groups) {
-    if (b.part) store_row<BLK>(b, nullptr);
-    return;
-  }
+  if (g_first >= n_groups) return;
   const uint32_t copy = blockIdx.x & (b.n_copies - 1u);
   const bool do_model = (stages & STAGE_MODEL) != 0;
   const bool do_contrib = (stages & STAGE_CONTRIB) != 0;
@@ -1250,10 +1245,7 @@ __global__ void __launch_bounds__(BLK)
     }
   }
   __syncthreads();
-  if (b.part)
-    store_row<BLK>(b, s_acc);
-  else
-    flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
+  flush_window<BLK>(s_acc, acc_S, acc_ns, acc_nc, acc_nc, 0u, tid);
 }
 
 // What the books read of a run, requested together (before its counter shards
@@ -2015,7 +2007,7 @@ static void launch_resolve(const BatchDev& b, int grid, uint32_t aux, bool ahead
 }
 template <class M>
 void resolve_t(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_t s) {
-  if (b.part)
+  if (b.rows)
     launch_resolve<M, TAKE_ROWS>(b, grid, aux, ahead, s);
   else if (b.n_copies == 1)
     launch_resolve<M, 1>(b, grid, aux, ahead, s);
@@ -2024,7 +2016,7 @@ void resolve_t(const BatchDev& b, int grid, uint32_t aux, bool ahead, hipStream_
 }
 template <class M>
 const void* resolve_kernel_t(const BatchDev& b) {
-  return b.part            ? (const void*)&k_resolve<M, TAKE_ROWS>
+  return b.rows            ? (const void*)&k_resolve<M, TAKE_ROWS>
          : b.n_copies == 1 ? (const void*)&k_resolve<M, 1>
                            : (const void*)&k_resolve<M, (int)run_copies(M::NS)>;
 }

@@ -15,7 +15,7 @@
 
 namespace mcst {
 
-constexpr uint32_t UDF_ABI_VERSION = 19;
+constexpr uint32_t UDF_ABI_VERSION = 20;
 
 struct UdfModel {
   uint32_t abi_version;
