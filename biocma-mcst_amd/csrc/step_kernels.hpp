@@ -1481,8 +1481,12 @@ __device__ __forceinline__ uint32_t request_prefix(const BatchDev& b, uint32_t s
   const uint32_t i2 = (a3 << 6) + lane, i1 = (b.moved ? 0u : a2 << 6) + lane, i0 = (a1 << 6) + lane;
   const uint32_t x2 = i2 < a2 ? b.div_l2[i2] : 0u;
   const uint32_t x0 = i0 < sc ? b.sub_divs[i0] : 0u;
-  uint32_t x1 = 0;  // one round but in a small pool
-  for (uint32_t i = i1; i < a1; i += 64) x1 += b.div_l1[i];
+  uint32_t x1 = i1 < a1 ? b.div_l1[i1] : 0u;
+  if (b.moved && a1 > 64u)
+    for (uint32_t i = i1 + 64u; i < a1; i += 256) {
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) x1 += i + 64 * k < a1 ? b.div_l1[i + 64 * k] : 0u;
+    }
   return wave_sum(v + x2 + x1 + x0);
 }
 
