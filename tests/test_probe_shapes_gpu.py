@@ -19,9 +19,18 @@ def shape(err):
 @pytest.mark.parametrize("block", [None, "512", "1024"])
 @pytest.mark.parametrize("network", ["whole", "window"])
 def test_probing_pass_has_its_own_shape(block, network, monkeypatch, capfd):
-    import torch
+    import mcst
 
     monkeypatch.setenv("MCST_VERBOSE", "1")
+    # the windowed pass without probes has one block of 1024 threads a compute unit
+    ref = mcst.Engine("quad_monod")
+    c = cases.lattice50k(n_particles=1000)
+    c.capacity = 600_000
+    c.apply(ref.add_run(c.n_c, c.dt, c.seed))
+    ref.commit()
+    one, cus, _, _ = shape(capfd.readouterr().err)
+    assert one == 1024
+    ref.close()
     if block:
         monkeypatch.setenv("MCST_PARTICLE_BLOCK", block)
     if network == "whole":
@@ -30,7 +39,6 @@ def test_probing_pass_has_its_own_shape(block, network, monkeypatch, capfd):
         c = cases.lattice50k(n_particles=100_000)
     eng, g, o = make_pair(c, capacity=600_000)
     blk, grid, lds, priv = shape(capfd.readouterr().err)
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert (blk, grid, priv) == (256, 2 * cus, 1)
     eng.step(3)
     o.step(3, threads=8)
