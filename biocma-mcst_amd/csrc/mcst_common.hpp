@@ -54,9 +54,10 @@ static_assert(TILE <= MOVER_INACTIVE, "a tile-local slot fits below the flag");
 // 1e6 29.4, 28.1, 42.0 and 30.6, 28.0, 41.0: the line.  Where the pipelined pass
 // holds many states of 4 slots per lane its registers leave it few waves and the
 // line lies further up: 6 states 1e6 34.5 and 34.7, 2e6 51.0 and 47.4, 3e6 64.2
-// and 59.7, 5e6 91.9 and 91.9; 9 states 1e6 50.6 and 47.0, 2e6 77.6 and 70-80,
-// 3e6 107 and 138, which a pool of these tiles holds only when it is full (its
-// slots are what is known here, and a run has twice its particles by default).
+// and 59.7, 5e6 91.9 and 91.9; 9 states (half as many again after their first
+// steps) 1e6 50.6 and 47.0, 2e6 77.6 and 70-80, 3e6 107 and 138, which a pool of
+// these tiles holds only when it is full (its slots are what is known here, and
+// a run has twice its particles by default).
 constexpr uint32_t small_tiles(int nv, int nl) { return nv * nl >= 24 ? 3072u : 1024u; }
 
 // Stage mask of one step (values shared with the C ABI).

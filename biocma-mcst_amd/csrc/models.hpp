@@ -157,7 +157,7 @@ constexpr int record_terms() {
 // WRITES (vars_declared_soundly): alone, zeros would be stored over variables
 // that were never loaded.  A variable that update() writes on some of its paths
 // only counts as read, too: its old value is stored on the others.  The particle pass loads the former, and stores the latter of the Idle
-// slots: with 4 + 6 values of 9 + 9 the pass of 1e6 simple_acetate cells takes
+// slots: with 4 + 6 values of 9 + 9 the pass of 1.5e6 simple_acetate cells takes
 // 31.4 us instead of 41.4, with 4 + 6 of 8 + 8 that of 1.2e7 quad_monod cells 324
 // instead of 375, with 2 + 1 of 2 + 2 that of 40 uneven runs 83.8 instead of
 // 92.5.  division() may use every variable: the pass loads the others for the

@@ -1836,8 +1836,8 @@ __device__ __forceinline__ void add_by_compartment(double* acc, bool in, uint32_
 // A block takes a contiguous range of slots and sums them in LDS, then adds
 // its nonzero sums to the device's: with one global atomic per particle and
 // variable instead, the particles of a compartment, which sit together, queued
-// on one address (1e6 particles of 10 values in 500 compartments 1187 us, now
-// 58 us; 1e5 of 3 in 64 compartments 234 us, now 17 us).  LDS holds `vg` variables of `win`
+// on one address (1.5e6 particles of 10 values in 500 compartments 1187 us, now
+// 56 us; 1e5 of 3 in 64 compartments 234 us, now 17 us).  LDS holds `vg` variables of `win`
 // compartments; block row y takes one such share (variables y % n_vg, window
 // y / n_vg), reading the positions again for each.
 constexpr uint32_t EXPORT_THREADS = 512;

@@ -286,7 +286,7 @@ int mcst_engine_profile(mcst_engine* e, uint32_t n_steps, double* total_ms, doub
 /* Autotuner of the particle pass (no counterpart in the reference; the
  * launch shapes of its Kokkos kernels are fixed).  Runs `steps` real steps
  * with each candidate shape (threads per block 256/512/1024 x consecutive
- * tiles per block turn 0/1/2/4/8), times the particle pass with HIP events,
+ * groups of tiles per block turn 0/1/2/4/8; 0/1 for the pass of small pools), times the particle pass with HIP events,
  * and keeps the fastest for the engine's later steps (also across admit and
  * retire); the untuned shape stays unless another is at least 2 % faster.  The runs advance by the trial steps; their results do not depend
  * on the shape.  Drops a captured graph. */
