@@ -1876,11 +1876,13 @@ __global__ void __launch_bounds__(EXPORT_THREADS) k_properties(BatchDev b, uint3
     const uint64_t mask = __ballot(in);
     const uint32_t lead = mask ? (uint32_t)__ffsll((long long)mask) - 1u : 0u;
     const uint32_t k0 = (uint32_t)__shfl((int)k, (int)lead, 64);
+    if (!mask && !store) continue;  // none of the wave's particles in this window
     const bool one = mask && __ballot(in && k == k0) == mask;
+    const bool need = live && (in || store);  // a particle's values are read in its own window only
     double x[NV];
 #pragma unroll
     for (uint32_t v = 0; v < NV; ++v)
-      x[v] = (has_mass || (v >= v0 && v < v1)) && live ? b.state[(uint64_t)v * b.P + g] : 0.0;
+      x[v] = (has_mass || (v >= v0 && v < v1)) && need ? b.state[(uint64_t)v * b.P + g] : 0.0;
 #pragma unroll
     for (uint32_t v = 0; v < NV; ++v) {
       if (v < v0 || v >= v1) continue;
@@ -1888,7 +1890,7 @@ __global__ void __launch_bounds__(EXPORT_THREADS) k_properties(BatchDev b, uint3
       add_by_compartment(s_acc + (v - v0) * w, in, k, one, k0, lane, x[v]);
     }
     if (has_mass) {
-      const double m = live ? M::mass(p, x) : 0.0;
+      const double m = need ? M::mass(p, x) : 0.0;
       if (store && valid) values[(uint64_t)NV * n + s] = m;
       add_by_compartment(s_acc + (NV - v0) * w, in, k, one, k0, lane, m);
     }
